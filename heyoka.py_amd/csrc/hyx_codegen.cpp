@@ -180,6 +180,36 @@ std::string lit(double v)
 namespace
 {
 
+// The step-size rule from the norms mx, mo, mom1 (max |x|, and of the orders p and p - 1) and
+// max_dt: declares h. The two roots are hyx_root (hyx_kmath.hip).
+static void step_size(std::ostringstream &o, int P)
+{
+    o << "    const double rnum = 1.0 / ((mx <= 1.0) ? 1.0 : mx);\n";
+    o << "    const double rho_o = hyx_root<" << P << ">(rnum, mo);\n";
+    o << "    const double rho_om1 = hyx_root<" << P - 1 << ">(rnum, mom1);\n";
+    o << "    const double rho_m = (rho_om1 < rho_o) ? rho_om1 : rho_o;\n";
+    const double e1 = std::exp(1.0);
+    const double rhofac = std::exp(-7.0 / 10.0 / (double)(P - 1)) / (e1 * e1);
+    o << "    double h = rho_m * " << lit(rhofac) << ";\n";
+    o << "    const double lim = fabs(max_dt);\n    h = (h < lim) ? h : lim;\n    if (max_dt < 0.0) h = -h;\n";
+}
+
+// c = a^al at order 0, declaring ra = 1 / a with it: by hyx_kmath.hip where it has the
+// exponent, else the library's pow().
+static void pow_order0(std::ostringstream &o, const std::string &c, const std::string &ra, const std::string &a, double al)
+{
+    if (al == -1.5 || al == -0.5) {
+        o << "    double " << ra << ";\n    const double " << c << " = " << (al == -1.5 ? "hyx_pow_m3_2(" : "hyx_pow_m1_2(")
+          << a << ", " << ra << ");\n";
+        return;
+    }
+    o << "    const double " << ra << " = 1.0 / " << a << ";\n    const double " << c << " = ";
+    if (al == -1.0)
+        o << ra << ";\n";
+    else
+        o << "pow(" << a << ", " << lit(al) << ");\n";
+}
+
 struct Gen {
     const Sys &S;
     const int P;
@@ -187,6 +217,7 @@ struct Gen {
     std::ostringstream o;
     std::set<std::pair<uint32_t, int>> zset; // (node, k) known to be exactly zero
     std::set<std::pair<uint32_t, int>> dvars; // generated j * a^[j] values
+    bool rhs_derivs = false;                  // the state variables' right-hand sides are nodes of this op-list
     std::vector<char> perlane;                // constants held per lane (kc_prefix[]) instead of literals
     std::string kc_prefix = "kc";
     // State coefficients in LDS: each lane keeps the rows x^[k] of its instance in
@@ -272,8 +303,10 @@ struct Gen {
     // j * a^[j], shared by the exp / sin / cos recurrences over the same argument.
     std::string dval(uint32_t w, int j)
     {
-        if (j == 1) return val(w, 1);
         const uint32_t idx = HYX_OPERAND_INDEX(w);
+        // j x^[j] of a state variable is the order j - 1 of its right-hand side.
+        if (rhs_derivs && idx < S.n && !zero(S.rhs[idx], j - 1)) return val(S.rhs[idx], j - 1);
+        if (j == 1) return val(w, 1);
         const std::string nm = "d" + std::to_string(idx) + "_" + std::to_string(j);
         if (!dvars.count({idx, j})) {
             dvars.insert({idx, j});
@@ -366,10 +399,9 @@ struct Gen {
             if (S.deg[j] > 0) o << "    const double rs" << j << " = 0.5 / " << c << ";\n";
             break;
         case HYX_OP_POW:
-            o << "    const double " << c << " = pow(" << v(0) << ", " << lit(S.consts[S.aux[j]]) << ");\n";
+            pow_order0(o, c, "ra" + std::to_string(j), v(0), S.consts[S.aux[j]]);
             if (S.deg[j] > 0) {
                 const double al = S.consts[S.aux[j]];
-                o << "    const double ra" << j << " = 1.0 / " << v(0) << ";\n";
                 o << "    const double raa" << j << " = ra" << j << " * " << lit(al) << ";\n";
                 o << "    const double rab" << j << " = ra" << j << " * " << lit(al + 1.0) << ";\n";
             }
@@ -684,6 +716,7 @@ struct Gen {
         };
         // order 0
         cur_k = 0;
+        rhs_derivs = true;
         for (uint32_t i = 0; i < n; ++i) {
             if (quad && qsig[i] != i)
                 o << "    const double " << cv(i, 0) << " = hyx_quad_y ? x[" << qsig[i] << "] : x[" << i << "];\n";
@@ -740,26 +773,17 @@ struct Gen {
             o << eg.o.str() << "    }\n";
         }
         // Step size: infinity norms of the state and of the last two orders.
-        o << "    double mx = 0.0, mo = 0.0, mom1 = 0.0, ab;\n";
+        o << "    double mx = 0.0, mo = 0.0, mom1 = 0.0;\n";
         for (uint32_t i = 0; i < n; ++i) {
-            o << "    ab = fabs(" << nv(i, 0) << "); mx = (ab > mx) ? ab : mx;\n";
-            o << "    ab = fabs(" << nv(i, P) << "); mo = (ab > mo) ? ab : mo;\n";
-            o << "    ab = fabs(" << nv(i, P - 1) << "); mom1 = (ab > mom1) ? ab : mom1;\n";
+            o << "    mx = fmax(mx, fabs(" << nv(i, 0) << "));\n";
+            o << "    mo = fmax(mo, fabs(" << nv(i, P) << "));\n";
+            o << "    mom1 = fmax(mom1, fabs(" << nv(i, P - 1) << "));\n";
         }
         for (uint32_t e = 0; E && e < nev; ++e) {
-            o << "    ab = fabs(hyx_evg[" << e << "][" << P << "]); mo = (ab > mo) ? ab : mo;\n";
-            o << "    ab = fabs(hyx_evg[" << e << "][" << (P - 1) << "]); mom1 = (ab > mom1) ? ab : mom1;\n";
+            o << "    mo = fmax(mo, fabs(hyx_evg[" << e << "][" << P << "]));\n";
+            o << "    mom1 = fmax(mom1, fabs(hyx_evg[" << e << "][" << (P - 1) << "]));\n";
         }
-        o << "    const double num = (mx <= 1.0) ? 1.0 : mx;\n";
-        o << "    const double rho_o = pow(num / mo, " << lit(1.0 / P) << ");\n";
-        o << "    const double rho_om1 = pow(num / mom1, " << lit(1.0 / (P - 1)) << ");\n";
-        o << "    const double rho_m = (rho_om1 < rho_o) ? rho_om1 : rho_o;\n";
-        const double e1 = std::exp(1.0);
-        const double rhofac = std::exp(-7.0 / 10.0 / (double)(P - 1)) / (e1 * e1);
-        o << "    double h = rho_m * " << lit(rhofac) << ";\n";
-        o << "    const double lim = fabs(max_dt);\n";
-        o << "    h = (h < lim) ? h : lim;\n";
-        o << "    if (max_dt < 0.0) h = -h;\n";
+        step_size(o, P);
         if (E) {
             // Fast exclusion per event over the step (the same test the root scan starts
             // with); only steps it cannot clear keep their coefficients in memory.
@@ -889,8 +913,8 @@ struct CompactGen {
             o << "    const double rs" << j << " = 0.5 / " << c << ";\n";
             break;
         case HYX_OP_POW:
-            o << "    " << c << " = pow(" << v0(A[0]) << ", " << lit(S.consts[S.aux[j]]) << ");\n";
-            o << "    const double ra" << j << " = 1.0 / " << v0(A[0]) << ";\n";
+            pow_order0(o, "p0_" + std::to_string(j), "ra" + std::to_string(j), v0(A[0]), S.consts[S.aux[j]]);
+            o << "    " << c << " = p0_" << j << ";\n";
             break;
         case HYX_OP_EXP: o << "    " << c << " = exp(" << v0(A[0]) << ");\n"; break;
         case HYX_OP_LOG:
@@ -1069,20 +1093,11 @@ struct CompactGen {
         o << "    double mx = 0.0, mo = 0.0, mom1 = 0.0;\n";
         o << "    for (int i = 0; i < HYX_N; ++i) {\n"
              "        double ab = fabs(T(i, 0)); mx = (ab > mx) ? ab : mx;\n"
-             "        ab = fabs(T(i, HYX_P)); mo = (ab > mo) ? ab : mo;\n"
-             "        ab = fabs(T(i, HYX_P - 1)); mom1 = (ab > mom1) ? ab : mom1;\n"
+             "        mo = fmax(mo, fabs(T(i, HYX_P)));\n"
+             "        mom1 = fmax(mom1, fabs(T(i, HYX_P - 1)));\n"
              "    }\n";
         if (events) o << "    hyx_ev_norms(tc, tcs, pv, t0, mo, mom1);\n";
-        o << "    const double num = (mx <= 1.0) ? 1.0 : mx;\n";
-        o << "    const double rho_o = pow(num / mo, " << lit(1.0 / P) << ");\n";
-        o << "    const double rho_om1 = pow(num / mom1, " << lit(1.0 / (P - 1)) << ");\n";
-        o << "    const double rho_m = (rho_om1 < rho_o) ? rho_om1 : rho_o;\n";
-        const double e1 = std::exp(1.0);
-        const double rhofac = std::exp(-7.0 / 10.0 / (double)(P - 1)) / (e1 * e1);
-        o << "    double h = rho_m * " << lit(rhofac) << ";\n";
-        o << "    const double lim = fabs(max_dt);\n";
-        o << "    h = (h < lim) ? h : lim;\n";
-        o << "    if (max_dt < 0.0) h = -h;\n";
+        step_size(o, P);
         o << "    bool nf = false;\n";
         o << "#pragma unroll\n    for (int i = 0; i < HYX_N; ++i) {\n";
         if (!high_acc) {
@@ -1886,28 +1901,21 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
                      << ";\n";
         o << eg.o.str() << "    }\n";
     }
-    o << "    double mx = 0.0, mo = 0.0, mom1 = 0.0, ab;\n";
+    o << "    double mx = 0.0, mo = 0.0, mom1 = 0.0;\n";
     for (int oo = 0; oo < own; ++oo) {
-        o << "    ab = fabs(" << xv(oo, 0) << "); mx = (ab > mx) ? ab : mx;\n";
-        o << "    ab = fabs(" << xv(oo, P) << "); mo = (ab > mo) ? ab : mo;\n";
-        o << "    ab = fabs(" << xv(oo, P - 1) << "); mom1 = (ab > mom1) ? ab : mom1;\n";
+        o << "    mx = fmax(mx, fabs(" << xv(oo, 0) << "));\n";
+        o << "    mo = fmax(mo, fabs(" << xv(oo, P) << "));\n";
+        o << "    mom1 = fmax(mom1, fabs(" << xv(oo, P - 1) << "));\n";
     }
     for (uint32_t e = 0; E && e < nev; ++e) {
-        o << "    ab = fabs(hyx_evg[" << e << "][" << P << "]); mo = (ab > mo) ? ab : mo;\n";
-        o << "    ab = fabs(hyx_evg[" << e << "][" << (P - 1) << "]); mom1 = (ab > mom1) ? ab : mom1;\n";
+        o << "    mo = fmax(mo, fabs(hyx_evg[" << e << "][" << P << "]));\n";
+        o << "    mom1 = fmax(mom1, fabs(hyx_evg[" << e << "][" << (P - 1) << "]));\n";
     }
     o << "#pragma unroll\n    for (int off = 1; off < HYX_G; off <<= 1) {\n"
-         "        ab = __shfl_xor(mx, off); mx = (ab > mx) ? ab : mx;\n"
-         "        ab = __shfl_xor(mo, off); mo = (ab > mo) ? ab : mo;\n"
-         "        ab = __shfl_xor(mom1, off); mom1 = (ab > mom1) ? ab : mom1;\n    }\n";
-    o << "    const double num = (mx <= 1.0) ? 1.0 : mx;\n";
-    o << "    const double rho_o = pow(num / mo, " << lit(1.0 / P) << ");\n";
-    o << "    const double rho_om1 = pow(num / mom1, " << lit(1.0 / (P - 1)) << ");\n";
-    o << "    const double rho_m = (rho_om1 < rho_o) ? rho_om1 : rho_o;\n";
-    const double e1 = std::exp(1.0);
-    const double rhofac = std::exp(-7.0 / 10.0 / (double)(P - 1)) / (e1 * e1);
-    o << "    double h = rho_m * " << lit(rhofac) << ";\n";
-    o << "    const double lim = fabs(max_dt);\n    h = (h < lim) ? h : lim;\n    if (max_dt < 0.0) h = -h;\n";
+         "        mx = fmax(mx, __shfl_xor(mx, off));\n"
+         "        mo = fmax(mo, __shfl_xor(mo, off));\n"
+         "        mom1 = fmax(mom1, __shfl_xor(mom1, off));\n    }\n";
+    step_size(o, P);
     if (E) {
         // The same fast exclusion as the lane forms; the coefficients of the steps it
         // cannot clear go to tc (event rows by every lane, identical values; state rows
@@ -3675,28 +3683,21 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
                      << ";\n";
         o << eg.o.str() << "    }\n";
     }
-    o << "    double mx = 0.0, mo = 0.0, mom1 = 0.0, ab;\n";
+    o << "    double mx = 0.0, mo = 0.0, mom1 = 0.0;\n";
     for (int oo = 0; oo < own; ++oo) {
-        o << "    ab = fabs(" << xv(oo, 0) << "); mx = (ab > mx) ? ab : mx;\n";
-        o << "    ab = fabs(" << xv(oo, P) << "); mo = (ab > mo) ? ab : mo;\n";
-        o << "    ab = fabs(" << xv(oo, P - 1) << "); mom1 = (ab > mom1) ? ab : mom1;\n";
+        o << "    mx = fmax(mx, fabs(" << xv(oo, 0) << "));\n";
+        o << "    mo = fmax(mo, fabs(" << xv(oo, P) << "));\n";
+        o << "    mom1 = fmax(mom1, fabs(" << xv(oo, P - 1) << "));\n";
     }
     for (uint32_t e = 0; E && e < nev; ++e) {
-        o << "    ab = fabs(hyx_evg[" << e << "][" << P << "]); mo = (ab > mo) ? ab : mo;\n";
-        o << "    ab = fabs(hyx_evg[" << e << "][" << (P - 1) << "]); mom1 = (ab > mom1) ? ab : mom1;\n";
+        o << "    mo = fmax(mo, fabs(hyx_evg[" << e << "][" << P << "]));\n";
+        o << "    mom1 = fmax(mom1, fabs(hyx_evg[" << e << "][" << (P - 1) << "]));\n";
     }
     o << "#pragma unroll\n    for (int off = 1; off < HYX_G; off <<= 1) {\n"
-         "        ab = __shfl_xor(mx, off); mx = (ab > mx) ? ab : mx;\n"
-         "        ab = __shfl_xor(mo, off); mo = (ab > mo) ? ab : mo;\n"
-         "        ab = __shfl_xor(mom1, off); mom1 = (ab > mom1) ? ab : mom1;\n    }\n";
-    o << "    const double num = (mx <= 1.0) ? 1.0 : mx;\n";
-    o << "    const double rho_o = pow(num / mo, " << lit(1.0 / P) << ");\n";
-    o << "    const double rho_om1 = pow(num / mom1, " << lit(1.0 / (P - 1)) << ");\n";
-    o << "    const double rho_m = (rho_om1 < rho_o) ? rho_om1 : rho_o;\n";
-    const double e1 = std::exp(1.0);
-    const double rhofac = std::exp(-7.0 / 10.0 / (double)(P - 1)) / (e1 * e1);
-    o << "    double h = rho_m * " << lit(rhofac) << ";\n";
-    o << "    const double lim = fabs(max_dt);\n    h = (h < lim) ? h : lim;\n    if (max_dt < 0.0) h = -h;\n";
+         "        mx = fmax(mx, __shfl_xor(mx, off));\n"
+         "        mo = fmax(mo, __shfl_xor(mo, off));\n"
+         "        mom1 = fmax(mom1, __shfl_xor(mom1, off));\n    }\n";
+    step_size(o, P);
     if (E) {
         const uint64_t off = (uint64_t)n * (P + 1) + (uint64_t)(E->nnodes - E->n) * (P + 1);
         o << "    hyx_evm = 0ull;\n";

@@ -31,7 +31,7 @@
 #include "../../include/hyx.h"
 #include "hyx_internal.h"
 
-#include "build/hyx_kernels_embed.inc" // k_hyx_kcommon, k_hyx_klane, k_hyx_kgroup, k_hyx_kcfunc, k_hyx_kevent: kernel templates
+#include "build/hyx_kernels_embed.inc" // k_hyx_kmath, k_hyx_kcommon, k_hyx_klane, k_hyx_kgroup, k_hyx_kcfunc, k_hyx_kevent: kernel templates
 
 namespace
 {
@@ -393,7 +393,7 @@ int build_sys(const uint32_t *ops, uint32_t n_words, const double *consts, uint3
         }
         if (s.form == HYX_FORM_GROUP || s.form == HYX_FORM_WAVE) {
             if (s.form == HYX_FORM_GROUP) s.inst_per_block = 64u / (uint32_t)gp.G;
-            s.src = (s.has_events ? hyx::events_forward_decl() : std::string()) +
+            s.src = std::string(k_hyx_kmath) + (s.has_events ? hyx::events_forward_decl() : std::string()) +
                     (s.form == HYX_FORM_WAVE
                          ? wave_src
                          : hyx::generate_group_prelude(s.S, gp, (int)order, ha, split, !(flags & HYX_FLAG_NO_PIPELINE),
@@ -421,9 +421,9 @@ int build_sys(const uint32_t *ops, uint32_t n_words, const double *consts, uint3
                 if (!(flags & HYX_FLAG_NO_QUAD)) tp = hyx::generate_quad_prelude(s.S, (int)order, ha, split, twhy);
                 s.tsub = tp.empty() ? 2 : 4;
                 if (tp.empty()) tp = hyx::generate_twin_prelude(s.S, (int)order, ha, split, twhy);
-                if (!tp.empty()) s.tsrc = tp + "\n" + k_hyx_kcommon + "\n" + k_hyx_klane;
+                if (!tp.empty()) s.tsrc = std::string(k_hyx_kmath) + tp + "\n" + k_hyx_kcommon + "\n" + k_hyx_klane;
             }
-            s.src = (s.has_events ? hyx::events_forward_decl() : std::string()) +
+            s.src = std::string(k_hyx_kmath) + (s.has_events ? hyx::events_forward_decl() : std::string()) +
                     hyx::generate_prelude(s.S, (int)order, ha, s.compact, split, sub, s.has_events ? &s.E : nullptr,
                                           (uint32_t)s.ev.dir.size(),
                                           (flags & HYX_FLAG_LDS_ROWS) ? 1 : (flags & HYX_FLAG_NO_LDS_ROWS) ? 0 : -1) +
@@ -587,7 +587,7 @@ int hyx_cfunc_create(const uint32_t *ops, uint32_t n_words, const double *consts
     c->n_in = n_in;
     c->n_out = n_out;
     try {
-        c->src = hyx::generate_cfunc_prelude(c->S, n_out) + "\n" + k_hyx_kcfunc;
+        c->src = std::string(k_hyx_kmath) + hyx::generate_cfunc_prelude(c->S, n_out) + "\n" + k_hyx_kcfunc;
     } catch (const std::exception &e) {
         return bad(HYX_EINVAL, e.what());
     }
