@@ -253,10 +253,17 @@ struct Gen {
     // the exchange changes which products the compiler would fuse.
     bool no_contract = false;
 
-    // Group form events: the state variables' coefficients are read from the LDS rows
-    // fl[lds_xb + k * lds_nx + lds_col[i]] (lds_xb < 0: not used).
-    int lds_xb = -1, lds_nx = 0;
-    std::vector<int> lds_col; // column of each state variable (empty: the variable's index)
+    // Group and wave form events: the state variables' coefficients are read from the LDS
+    // rows, by this expression for (variable, order).
+    std::function<std::string(uint32_t, int)> lds_row;
+
+    // Group form: the sums of products take their terms oldest first, and the terms without
+    // an order-k factor can be summed before the order's exchange has arrived (pre_order).
+    // Squares that only one sum reads (a distance) are summed as one chain with it.
+    bool newest_last = false;
+    std::map<uint32_t, std::vector<uint32_t>> sumsq; // sum node -> its squares
+    std::set<uint32_t> absorbed;                     // those squares
+    std::map<std::pair<uint32_t, int>, size_t> pre;  // terms of (node, order) already summed
 
     Gen(const Sys &s, int p, bool ha) : S(s), P(p), high_acc(ha), perlane(s.nconsts, 0) {}
 
@@ -267,8 +274,7 @@ struct Gen {
     // Coefficient k of node idx: a register, or for a state variable in LDS an older row.
     std::string nv(uint32_t idx, int k) const
     {
-        if (lds_xb >= 0 && idx < S.n)
-            return "fl[" + std::to_string(lds_xb + k * lds_nx + (lds_col.empty() ? (int)idx : lds_col[idx])) + "]";
+        if (lds_row && idx < S.n) return lds_row(idx, k);
         if (base && idx < base->S.n) return base->nv(idx, k);
         if (lds_state && idx < S.n && k != cur_k) return xs(idx, k);
         return cv(idx, k);
@@ -469,9 +475,129 @@ struct Gen {
           << val(w, k) << ");\n";
     }
 
+    // Group form, inputs x with x' = v that only linear nodes over inputs read: c<input>_<k> is
+    // v^[k-1], and the linear node (a difference of positions) multiplies by 1 / k, once.
+    bool raw_inputs = false;
+    bool reads_inputs(uint32_t j) const
+    {
+        for (auto a : S.args[j])
+            if (HYX_OPERAND_KIND(a) != HYX_KIND_NODE || HYX_OPERAND_INDEX(a) >= S.n) return false;
+        return S.op[j] == HYX_OP_ADD || S.op[j] == HYX_OP_SUB || S.op[j] == HYX_OP_NEG || S.op[j] == HYX_OP_SUM;
+    }
+    bool inputs_only_linear() const
+    {
+        for (uint32_t j = S.n; j < S.nnodes; ++j)
+            for (auto a : S.args[j])
+                if (HYX_OPERAND_KIND(a) == HYX_KIND_NODE && HYX_OPERAND_INDEX(a) < S.n && !reads_inputs(j)) return false;
+        return true;
+    }
+
+    // The terms of a product, a (sum of) squares (the products below the diagonal) or a pow
+    // at order k, those without an order-k factor first and the latest factor last.
+    struct Prod {
+        double cf;
+        std::string a, b;
+        int key;
+    };
+    std::vector<Prod> products(uint32_t j, int k, size_t &old) const
+    {
+        std::vector<Prod> t;
+        auto key = [&](int hi, uint32_t node) { return hi < k ? hi * (int)S.nnodes : k * (int)S.nnodes + (int)node; };
+        const auto &A = S.args[j];
+        const auto sq = sumsq.find(j);
+        if (sq != sumsq.end() || S.op[j] == HYX_OP_SQUARE) {
+            for (uint32_t s : sq != sumsq.end() ? sq->second : std::vector<uint32_t>{j}) {
+                const uint32_t w = S.args[s][0];
+                for (int q = 0; 2 * q < k; ++q)
+                    if (!zero(w, q) && !zero(w, k - q))
+                        t.push_back({1.0, val(w, q), val(w, k - q), key(k - q, HYX_OPERAND_INDEX(w))});
+            }
+        } else if (S.op[j] == HYX_OP_POW) {
+            const double al = S.consts[S.aux[j]];
+            for (int q = 0; q < k; ++q) {
+                const double cf = (double)k * al - (double)q * (al + 1.0);
+                if (!zero(A[0], k - q) && cf != 0.0)
+                    t.push_back({cf, val(A[0], k - q), cv(j, q), key(std::max(q, k - q), HYX_OPERAND_INDEX(A[0]))});
+            }
+        } else
+            for (int q = 0; q <= k; ++q)
+                if (!zero(A[0], q) && !zero(A[1], k - q))
+                    t.push_back({1.0, val(A[0], q), val(A[1], k - q),
+                                 key(std::max(q, k - q), HYX_OPERAND_INDEX(q == k ? A[0] : A[1]))});
+        std::stable_sort(t.begin(), t.end(), [](const Prod &x, const Prod &y) { return x.key < y.key; });
+        old = 0;
+        while (old < t.size() && t[old].key < k * (int)S.nnodes) ++old;
+        return t;
+    }
+
+    bool sums_products(uint32_t j) const
+    {
+        if (!newest_last || absorbed.count(j)) return false;
+        if (sumsq.count(j) || S.op[j] == HYX_OP_SQUARE) return true;
+        if (S.op[j] == HYX_OP_POW) return literal_pow && short_pow_coeffs(S.consts[S.aux[j]]);
+        return S.op[j] == HYX_OP_MUL && !scalar(S.args[j][0]) && !scalar(S.args[j][1]);
+    }
+
+    void add_products(const std::vector<Prod> &t, const std::string &nm, size_t from, size_t to)
+    {
+        for (size_t q = from; q < to; ++q) {
+            const std::string f = t[q].cf == 1.0 ? t[q].a : lit(t[q].cf);
+            const std::string g = t[q].cf == 1.0 ? t[q].b : "(" + t[q].a + " * " + t[q].b + ")";
+            if (q == 0)
+                o << "    double " << nm << " = " << f << " * " << g << ";\n";
+            else
+                o << "    " << nm << " = __builtin_fma(" << f << ", " << g << ", " << nm << ");\n";
+        }
+    }
+
+    static std::string sum_name(uint32_t j, int k) { return "a" + std::to_string(j) + "_" + std::to_string(k); }
+
+    // The part of node j's order k that reads orders below k only.
+    void pre_order(uint32_t j, int k)
+    {
+        if (k > S.deg[j] || !sums_products(j)) return;
+        size_t old;
+        const auto t = products(j, k, old);
+        add_products(t, sum_name(j, k), 0, old);
+        pre[{j, k}] = old;
+    }
+
     void orderk(uint32_t j, int k)
     {
         if (k > S.deg[j]) return; // zero by degree; never referenced
+        if (absorbed.count(j)) return;
+        if (sums_products(j)) {
+            size_t old;
+            const auto t = products(j, k, old);
+            const std::string nm = sum_name(j, k), c = cv(j, k);
+            const auto pr = pre.find({j, k});
+            add_products(t, nm, pr == pre.end() ? 0 : pr->second, t.size());
+            const auto sq = sumsq.find(j);
+            if (sq != sumsq.end() || S.op[j] == HYX_OP_SQUARE) {
+                // Twice the terms below the diagonal, plus the diagonal's.
+                std::string d;
+                for (uint32_t s : sq != sumsq.end() ? sq->second : std::vector<uint32_t>{j}) {
+                    const uint32_t w = S.args[s][0];
+                    if (k % 2 || zero(w, k / 2)) continue;
+                    const std::string v = val(w, k / 2);
+                    d = d.empty() ? v + " * " + v : "__builtin_fma(" + v + ", " + v + ", " + d + ")";
+                }
+                if (t.empty() && d.empty())
+                    set_zero(j, k);
+                else if (t.empty())
+                    o << "    const double " << c << " = " << d << ";\n";
+                else if (d.empty())
+                    o << "    const double " << c << " = " << nm << " + " << nm << ";\n";
+                else
+                    o << "    const double " << c << " = __builtin_fma(2.0, " << nm << ", " << d << ");\n";
+            } else if (t.empty())
+                set_zero(j, k);
+            else if (S.op[j] == HYX_OP_POW)
+                o << "    const double " << c << " = " << nm << " * (ra" << j << " * " << lit(1.0 / k) << ");\n";
+            else
+                o << "    const double " << c << " = " << nm << ";\n";
+            return;
+        }
         const auto &A = S.args[j];
         const std::string c = cv(j, k);
         const std::string ks = std::to_string(k);
@@ -494,6 +620,8 @@ struct Gen {
             }
             if (first)
                 set_zero(j, k);
+            else if (raw_inputs && reads_inputs(j))
+                o << "    const double " << c << " = (" << e << ") * " << lit(1.0 / k) << ";\n";
             else
                 o << "    const double " << c << " = " << e << ";\n";
             break;
@@ -643,6 +771,30 @@ struct Gen {
             break;
         case HYX_OP_TWIN_XCH: xch(j, k); break;
         case HYX_OP_QUAD_SWAP: qswap(j, k); break;
+        }
+    }
+
+    // Finds the sums whose operands are all squares that nothing else reads (outs: nodes
+    // read outside the op-list).
+    void find_sumsq(const std::vector<uint32_t> &outs)
+    {
+        std::vector<int> uses(S.nnodes, 0);
+        for (uint32_t j = S.n; j < S.nnodes; ++j)
+            for (auto a : S.args[j])
+                if (HYX_OPERAND_KIND(a) == HYX_KIND_NODE) ++uses[HYX_OPERAND_INDEX(a)];
+        for (auto j : outs) uses[j] += 2;
+        for (uint32_t j = S.n; j < S.nnodes; ++j) {
+            if (S.op[j] != HYX_OP_SUM && S.op[j] != HYX_OP_ADD) continue;
+            std::vector<uint32_t> sq;
+            for (auto a : S.args[j]) {
+                const uint32_t idx = HYX_OPERAND_INDEX(a);
+                if (HYX_OPERAND_KIND(a) == HYX_KIND_NODE && idx >= S.n && S.op[idx] == HYX_OP_SQUARE && uses[idx] == 1 &&
+                    !scalar(S.args[idx][0]))
+                    sq.push_back(idx);
+            }
+            if (sq.size() != S.args[j].size()) continue;
+            sumsq[j] = sq;
+            absorbed.insert(sq.begin(), sq.end());
         }
     }
 
@@ -1150,7 +1302,10 @@ bool is_linear(uint32_t op) { return op == HYX_OP_ADD || op == HYX_OP_SUB || op 
 
 } // namespace
 
-bool plan_groups(const Sys &S, GroupPlan &gp, std::string &why)
+// fold: a product of a number and a node that only right-hand sides read is no node of its
+// cluster but a scale of the right-hand sides' terms (the masses of an N-body problem: three
+// outputs per pair instead of six, and the owners' sums are fma chains instead of sums).
+static bool plan_groups_impl(const Sys &S, GroupPlan &gp, std::string &why, bool pipeline, bool fold)
 {
     const uint32_t n = S.n, NN = S.nnodes;
     if (NN == n) {
@@ -1192,6 +1347,25 @@ bool plan_groups(const Sys &S, GroupPlan &gp, std::string &why)
             if (HYX_OPERAND_KIND(a) == HYX_KIND_NODE && internal[HYX_OPERAND_INDEX(a)]) {
                 why = "a linear right-hand-side node is also used inside a cluster";
                 return false;
+            }
+    }
+    if (fold) {
+        std::vector<char> used(NN, 0);
+        for (uint32_t j = n; j < NN; ++j)
+            if (!internal[j])
+                for (auto a : S.args[j])
+                    if (HYX_OPERAND_KIND(a) == HYX_KIND_NODE) used[HYX_OPERAND_INDEX(a)] = 1;
+        for (uint32_t i = 0; i < n; ++i)
+            for (auto &t : terms[i]) {
+                const uint32_t idx = HYX_OPERAND_INDEX(t.first);
+                if (HYX_OPERAND_KIND(t.first) != HYX_KIND_NODE || idx < n || used[idx] || S.op[idx] != HYX_OP_MUL) continue;
+                uint32_t c = S.args[idx][0], in = S.args[idx][1];
+                if (HYX_OPERAND_KIND(c) != HYX_KIND_CONST) std::swap(c, in);
+                if (HYX_OPERAND_KIND(c) != HYX_KIND_CONST || HYX_OPERAND_KIND(in) != HYX_KIND_NODE ||
+                    HYX_OPERAND_INDEX(in) < n || internal[HYX_OPERAND_INDEX(in)])
+                    continue;
+                internal[idx] = 1;
+                t = {in, t.second * S.consts[HYX_OPERAND_INDEX(c)]};
             }
     }
     UF uf(NN);
@@ -1283,17 +1457,47 @@ bool plan_groups(const Sys &S, GroupPlan &gp, std::string &why)
         why = "more than 64 clusters";
         return false;
     }
-    const int own = (int)((n + G - 1) / G);
-    if (own > 8) {
+    if ((n + G - 1) / G > 8) {
         why = "too many state variables per lane";
         return false;
     }
+    // Derived variables: x' = v alone, v not derived itself and the source of no other, x read
+    // by no right-hand side; used when every cluster input is one.
+    std::vector<int> dsrc(n, -1);
+    {
+        auto lone = [&](uint32_t i) {
+            return terms[i].size() == 1 && HYX_OPERAND_INDEX(terms[i][0].first) < n && terms[i][0].second == 1.0 &&
+                   rconst[i] == 0.0;
+        };
+        std::vector<char> read(n, 0), taken(n, 0);
+        for (uint32_t i = 0; i < n; ++i)
+            for (auto &t : terms[i])
+                if (HYX_OPERAND_INDEX(t.first) < n) read[HYX_OPERAND_INDEX(t.first)] = 1;
+        for (uint32_t i = 0; i < n; ++i) {
+            if (!lone(i) || read[i]) continue;
+            const uint32_t v = HYX_OPERAND_INDEX(terms[i][0].first);
+            if (lone(v) || taken[v]) continue;
+            dsrc[i] = (int)v;
+            taken[v] = 1;
+        }
+        bool all = pipeline && !B[0].inputs.empty();
+        for (auto &b : B)
+            for (uint32_t v : b.inputs) all = all && dsrc[v] >= 0;
+        if (!all) dsrc.assign(n, -1);
+    }
+    std::vector<uint32_t> order;
+    for (uint32_t v = 0; v < n; ++v)
+        if (dsrc[v] < 0) order.push_back(v);
+    const bool derived = order.size() < n;
+    const int own_a = (int)((order.size() + G - 1) / G), own = derived ? 2 * own_a : own_a;
     gp = GroupPlan{};
     gp.G = G;
     gp.ncl = ncl;
     gp.nin = (int)B[0].inputs.size();
     gp.nout = (int)B[0].outs.size();
     gp.own = own;
+    gp.own_a = own_a;
+    gp.dsrc = dsrc;
     // Template: cluster 0 with inputs as state variables 0..nin-1.
     {
         Sys &T = gp.tmpl;
@@ -1348,6 +1552,12 @@ bool plan_groups(const Sys &S, GroupPlan &gp, std::string &why)
         for (size_t q = 0; q < B[c].kconsts.size(); ++q) gp.kc[(size_t)c * gp.nkc + q] = S.consts[B[c].kconsts[q]];
         for (size_t q = B[c].kconsts.size(); q < gp.tmpl.nconsts; ++q) gp.kc[(size_t)c * gp.nkc + q] = gp.tmpl.consts[q];
     }
+    // Lanes without a cluster evaluate the first one again, into output slots that nobody reads
+    // (on zeros they would meet its singularities, and the slow paths of its functions).
+    for (int c = ncl; c < G; ++c) {
+        std::copy_n(gp.iv.begin(), gp.nin, gp.iv.begin() + (size_t)c * std::max(gp.nin, 1));
+        std::copy_n(gp.kc.begin(), gp.nkc, gp.kc.begin() + (size_t)c * gp.nkc);
+    }
     // Output q of lane c lives at LDS index q * (G + 1) + c: the lanes of a group write
     // one output row with consecutive 8-byte words, and the odd row stride puts the
     // outputs of one cluster in different banks, so owners summing several outputs of
@@ -1359,11 +1569,10 @@ bool plan_groups(const Sys &S, GroupPlan &gp, std::string &why)
         for (size_t q = 0; q < B[c].outs.size(); ++q) outslot[B[c].outs[q]] = (int)q * OS + c;
     // Ownership: variables sorted by (output terms, state terms), dealt to lanes slot
     // by slot, so that each slot's term counts are as uniform as possible.
-    std::vector<uint32_t> order(n);
-    std::vector<int> n_out(n, 0), n_st(n, 0);
+    std::vector<int> n_out(n, 0), n_st(n, 0), deriv(n, -1);
     for (uint32_t v = 0; v < n; ++v) {
-        order[v] = v;
         for (auto &t : terms[v]) (HYX_OPERAND_INDEX(t.first) < n ? n_st[v] : n_out[v])++;
+        if (dsrc[v] >= 0) deriv[dsrc[v]] = (int)v;
     }
     std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
         return std::make_pair(n_out[a], n_st[a]) > std::make_pair(n_out[b], n_st[b]);
@@ -1372,46 +1581,57 @@ bool plan_groups(const Sys &S, GroupPlan &gp, std::string &why)
     gp.rc.assign((size_t)G * own, 0.0);
     gp.nto.assign(own, 0);
     gp.nts.assign(own, 0);
-    for (uint32_t i = 0; i < n; ++i) {
-        const uint32_t v = order[i];
-        const int g = (int)(i % G), o = (int)(i / G);
-        gp.vo[(size_t)g * own + o] = (int)v;
-        gp.rc[(size_t)g * own + o] = rconst[v];
-        gp.nto[o] = std::max(gp.nto[o], n_out[v]);
-        gp.nts[o] = std::max(gp.nts[o], n_st[v]);
-    }
     gp.tio.assign(own, {});
     gp.tis.assign(own, {});
     gp.tso.assign(own, {});
     gp.tss.assign(own, {});
-    for (int o = 0; o < own; ++o) {
-        gp.tio[o].assign((size_t)G * gp.nto[o], OS * gp.nout);
-        gp.tso[o].assign((size_t)G * gp.nto[o], 1.0);
-        gp.tis[o].assign((size_t)G * gp.nts[o], (int)n);
-        gp.tss[o].assign((size_t)G * gp.nts[o], 1.0);
-    }
-    for (int g = 0; g < G; ++g)
-        for (int o = 0; o < own; ++o) {
-            const int v = gp.vo[(size_t)g * own + o];
-            if (v < 0) continue;
+    for (int o = 0; o < own_a; ++o) {
+        const int i0 = o * G, cnt = std::min<int>(G, (int)order.size() - i0);
+        int nto = 0, nts = 0;
+        for (int i = 0; i < cnt; ++i) {
+            nto = std::max(nto, n_out[order[i0 + i]]);
+            nts = std::max(nts, n_st[order[i0 + i]]);
+        }
+        gp.nto[o] = nto;
+        gp.nts[o] = nts;
+        gp.tio[o].assign((size_t)G * nto, OS * gp.nout);
+        gp.tso[o].assign((size_t)G * nto, 1.0);
+        gp.tis[o].assign((size_t)G * nts, (int)n);
+        gp.tss[o].assign((size_t)G * nts, 1.0);
+        for (int i = 0; i < cnt; ++i) {
+            const uint32_t v = order[i0 + i];
             int a = 0, b = 0;
+            gp.vo[(size_t)i * own + o] = (int)v;
+            gp.rc[(size_t)i * own + o] = rconst[v];
+            if (derived) gp.vo[(size_t)i * own + own_a + o] = deriv[v];
             for (auto &t : terms[v]) {
                 const uint32_t idx = HYX_OPERAND_INDEX(t.first);
                 if (idx < n) {
-                    gp.tis[o][(size_t)g * gp.nts[o] + b] = (int)idx;
-                    gp.tss[o][(size_t)g * gp.nts[o] + b] = t.second;
+                    gp.tis[o][(size_t)i * nts + b] = (int)idx;
+                    gp.tss[o][(size_t)i * nts + b] = t.second;
                     ++b;
                 } else {
                     if (outslot[idx] < 0) {
                         why = "a right-hand-side term is not a cluster output";
                         return false;
                     }
-                    gp.tio[o][(size_t)g * gp.nto[o] + a] = outslot[idx];
-                    gp.tso[o][(size_t)g * gp.nto[o] + a] = t.second;
+                    gp.tio[o][(size_t)i * nto + a] = outslot[idx];
+                    gp.tso[o][(size_t)i * nto + a] = t.second;
                     ++a;
                 }
             }
         }
+    }
+    return true;
+}
+
+bool plan_groups(const Sys &S, GroupPlan &gp, std::string &why, bool pipeline)
+{
+    // The form applies where the clusters with all their nodes are isomorphic.
+    if (!plan_groups_impl(S, gp, why, pipeline, false)) return false;
+    GroupPlan f;
+    std::string w;
+    if (plan_groups_impl(S, f, w, pipeline, true)) gp = f;
     return true;
 }
 
@@ -1560,28 +1780,66 @@ static OutputSlots lds_output_map(int G, int OS, int nout, const std::vector<std
     return best < base ? cur : m;
 }
 
+// The value of v in the other half of a block of 2 OFF lanes, for v alike within halves
+// (the steps of a sum or maximum over a group): DPP moves up to 16 lanes, one instruction
+// per 32 bits, instead of a trip through the LDS crossbar. hyx_gany: any lane's v non-zero.
+static std::string group_fold_src()
+{
+    return "#ifdef HYX_CPU_EMU\n"
+           "template <int OFF>\nstatic double hyx_gfold(double v) { return __shfl_xor(v, OFF); }\n"
+           "template <int OFF>\nstatic int hyx_gfold(int v) { return __shfl_xor(v, OFF); }\n"
+           "#else\n"
+           "template <int OFF>\n__device__ __forceinline__ int hyx_gfold(int v)\n{\n"
+           "    // quad_perm [1, 0, 3, 2], quad_perm [2, 3, 0, 1], row_half_mirror, row_mirror\n"
+           "    if constexpr (OFF < 16)\n"
+           "        return __builtin_amdgcn_update_dpp(0, v, OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : OFF == 4 ? 0x141 : 0x140, 0xF, 0xF, true);\n"
+           "    else\n        return __shfl_xor(v, OFF);\n}\n"
+           "template <int OFF>\n__device__ __forceinline__ double hyx_gfold(double v)\n{\n"
+           "    const hyx_u64 b = __builtin_bit_cast(hyx_u64, v);\n"
+           "    const int lo = hyx_gfold<OFF>((int)(unsigned)b), hi = hyx_gfold<OFF>((int)(unsigned)(b >> 32));\n"
+           "    return __builtin_bit_cast(double, ((hyx_u64)(unsigned)hi << 32) | (hyx_u64)(unsigned)lo);\n}\n"
+           "#endif\n"
+           "template <int OFF = 1>\n__device__ __forceinline__ int hyx_gany(int v)\n{\n"
+           "    if constexpr (OFF < HYX_G) return hyx_gany<2 * OFF>(v | hyx_gfold<OFF>(v));\n    else return v;\n}\n";
+}
+
+// The norms over the lanes of the group.
+static void group_norms(std::ostringstream &o, int G)
+{
+    for (int off = 1; off < G; off <<= 1)
+        for (const char *v : {"mx", "mo", "mom1"})
+            o << "    " << v << " = fmax(" << v << ", hyx_gfold<" << off << ">(" << v << "));\n";
+}
+
 std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, bool high_acc, int split_min,
                                    bool pipeline, const Sys *E, uint32_t nev)
 {
     const int G = gp.G, own = gp.own, nin = gp.nin, nout = gp.nout;
-    const int n = (int)S.n, nx = n + 1;
+    const int n = (int)S.n, own_a = gp.own_a;
+    const bool derived = own_a < own;
     const int OS = gp.os; // output row stride of the identity layout (the tio tables)
     std::vector<std::pair<std::vector<int>, int>> oreads;
-    for (int o = 0; o < own; ++o)
+    for (int o = 0; o < own_a; ++o)
         for (int t = 0; t < gp.nto[o]; ++t) {
             std::vector<int> as;
             for (int g = 0; g < G; ++g) as.push_back(gp.tio[o][(size_t)g * gp.nto[o] + t]);
             oreads.push_back({as, P});
         }
     const OutputSlots oslot = lds_output_map(G, OS, nout, oreads);
-    const int xb = std::max(oslot.zero, OS) + 1; // LDS: outputs, zero slot, then x[P+1][n+1]
-    const int flat = xb + (P + 1) * nx;
+    // LDS: outputs, zero slot, then the x rows: order 0 of every variable (nx columns), orders
+    // 1 .. P of the variables that are not derived (rs columns each, one of them zero).
+    int na = 0;
+    for (int v = 0; v < n; ++v) na += gp.dsrc[(size_t)v] < 0;
+    const int xb = std::max(oslot.zero, OS) + 1, rs = na + 1, nx = derived ? 2 * rs : rs;
+    const int flat = xb + nx + P * rs;
     std::ostringstream h;
     h << "#define HYX_N " << n << "\n#define HYX_NPAR " << std::max<uint32_t>(S.npar, 1) << "\n#define HYX_P " << P
       << "\n#define HYX_GROUP 1\n#define HYX_G " << G << "\n#define HYX_I " << (64 / G) << "\n#define HYX_NIN "
       << std::max(nin, 1) << "\n#define HYX_NOUT " << std::max(nout, 1) << "\n#define HYX_NKC " << gp.nkc
-      << "\n#define HYX_OWN " << own << "\n#define HYX_NX " << nx << "\n#define HYX_XB " << xb << "\n#define HYX_FLAT "
-      << flat << "\n";
+      << "\n#define HYX_OWN " << own << "\n#define HYX_NX " << nx << "\n#define HYX_RS " << rs << "\n#define HYX_XB " << xb
+      << "\n#define HYX_FLAT " << flat << "\n";
+    h << "#define HYX_VO(o) hyx_tab_vo[g * HYX_OWN + (o)]\n";
+    if ((long)(flat + 14) * (64 / G) * 8 > 160 * 1024) h << "#define HYX_REC_REGS 1\n";
     h << "typedef unsigned long long hyx_u64;\n";
     h << "#ifndef HYX_CPU_EMU\n"
          "// A block is one wavefront, and the LDS operations of a wavefront complete in issue\n"
@@ -1593,6 +1851,7 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
          "    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");\n}\n"
          "#define HYX_EMU_SYNC() hyx_wsync()\n"
          "#endif\n";
+    h << group_fold_src();
     auto itab = [&](const std::string &nm, const std::vector<int> &v) {
         h << "__constant__ int " << nm << "[" << std::max<size_t>(v.size(), 1) << "] = {";
         for (size_t q = 0; q < v.size(); ++q) h << (q ? "," : "") << v[q];
@@ -1610,7 +1869,7 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
     // the state terms (variable, scale) of that right-hand side, in the owner's order.
     std::vector<std::pair<int, int>> owner(n, {-1, -1});
     for (int g = 0; g < G; ++g)
-        for (int oo = 0; oo < own; ++oo) {
+        for (int oo = 0; oo < own_a; ++oo) {
             const int v = gp.vo[(size_t)g * own + oo];
             if (v >= 0 && v < n) owner[v] = {g, oo};
         }
@@ -1619,6 +1878,7 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
     for (int g = 0; g < G && lagged; ++g)
         for (int q = 0; q < nin && lagged; ++q) {
             const int v = gp.iv[(size_t)g * nin + q];
+            if (derived) continue; // every input is a derived variable
             if (v < 0 || v >= n || owner[v].first < 0) {
                 lagged = false;
                 break;
@@ -1628,6 +1888,7 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
                 if (gp.tio[oo][(size_t)g2 * gp.nto[oo] + t] != OS * nout) lagged = false;
             nls = std::max(nls, gp.nts[oo]);
         }
+    if (derived) nls = 1;
     if (nls == 0) lagged = false;
     std::vector<int> lis;
     std::vector<double> lss, lrc;
@@ -1640,6 +1901,10 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
         for (int g = 0; g < G; ++g)
             for (int q = 0; q < nin; ++q) {
                 const int v = gp.iv[(size_t)g * nin + q];
+                if (derived) {
+                    lis[(size_t)g * nin + q] = gp.dsrc[(size_t)v];
+                    continue;
+                }
                 const int g2 = owner[v].first, oo = owner[v].second;
                 for (int t = 0; t < gp.nts[oo]; ++t) {
                     lis[((size_t)g * nin + q) * nls + t] = gp.tis[oo][(size_t)g2 * gp.nts[oo] + t];
@@ -1659,25 +1924,34 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
     h << "#define HYX_PIPELINED " << (lagged ? 1 : 0) << "\n";
     // Column reads of one step, per group: the owners' rows (initial write, Horner, the
     // coefficient log), the cluster inputs (lagged: their state terms), the owners' state
-    // terms.
+    // terms. Columns are given to the variables that are not derived (aidx: their indices);
+    // the order-0 column of a derived variable is rs past its source's.
+    std::vector<int> aidx((size_t)n + 1, -1);
+    for (int v = 0, i = 0; v < n; ++v)
+        if (gp.dsrc[(size_t)v] < 0) aidx[(size_t)v] = i++;
+    aidx[(size_t)n] = na;
     std::vector<std::pair<std::vector<int>, int>> creads;
-    auto add_reads = [&](const std::vector<int> &tabv, int cnt, int weight) {
+    auto add_reads = [&](const std::vector<int> &tabv, int stride, int cnt, int weight) {
         for (int q = 0; q < cnt; ++q) {
             std::vector<int> vs;
             for (int g = 0; g < G; ++g) {
-                const int v = tabv[(size_t)g * cnt + q];
-                vs.push_back(v >= 0 && v < n ? v : n);
+                const int v = tabv[(size_t)g * stride + q];
+                vs.push_back(aidx[(size_t)(v >= 0 && v < n ? v : n)]);
             }
             creads.push_back({vs, weight});
         }
     };
-    add_reads(gp.vo, own, P + 3);
+    add_reads(gp.vo, own, own_a, P + 3);
     if (lagged)
-        add_reads(lis, nin * nls, P);
+        add_reads(lis, nin * nls, nin * nls, P);
     else
-        add_reads(gp.iv, nin, P + 1);
-    for (int o = 0; o < own; ++o) add_reads(gp.tis[o], gp.nts[o], P + 1);
-    const std::vector<int> col = lds_column_map(n, G, creads);
+        add_reads(gp.iv, nin, nin, P + 1);
+    for (int o = 0; o < own_a; ++o) add_reads(gp.tis[o], gp.nts[o], gp.nts[o], P + 1);
+    const std::vector<int> acol = lds_column_map(na, G, creads);
+    std::vector<int> col((size_t)n + 1);
+    for (int v = 0; v <= n; ++v)
+        col[(size_t)v] = aidx[(size_t)v] >= 0 ? acol[(size_t)aidx[(size_t)v]]
+                                              : rs + acol[(size_t)aidx[(size_t)gp.dsrc[(size_t)v]]];
     auto cols = [&](const std::vector<int> &tabv) {
         std::vector<int> r(tabv.size());
         for (size_t q = 0; q < tabv.size(); ++q) r[q] = col[(size_t)(tabv[q] >= 0 && tabv[q] < n ? tabv[q] : n)];
@@ -1706,6 +1980,7 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
         itab("hyx_tab_tis" + std::to_string(o), cols(gp.tis[o]));
         dtab("hyx_tab_tso" + std::to_string(o), gp.tso[o]);
         dtab("hyx_tab_tss" + std::to_string(o), gp.tss[o]);
+        if (o >= own_a) continue;
         auto uni = [&](const std::vector<double> &v, int cnt, int t, const std::string &arr) {
             bool same = true;
             for (int g = 1; g < G; ++g) same = same && v[(size_t)g * cnt + t] == v[t];
@@ -1748,18 +2023,44 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
     }
     h << "}\n";
 
+    // Coefficient k of the variable in slot o, from the rows.
+    std::vector<double> inv((size_t)P + 1, 1.0);
+    for (int k = 1; k <= P; ++k) inv[(size_t)k] = 1.0 / k;
+    dtab("hyx_tab_inv", inv);
+    h << "__device__ __forceinline__ double hyx_grow(const double *fl, const hyx_gtab &t, int o, int k)\n{\n";
+    if (derived)
+        h << "    if (o >= " << own_a << ") {\n        if (k == 0) return fl[HYX_XB + t.vc[o]];\n"
+             "        o -= " << own_a << ";\n        --k;\n"
+             "        return fl[(k == 0 ? HYX_XB : HYX_XB + HYX_NX + (k - 1) * HYX_RS) + t.vc[o]] * hyx_tab_inv[k + 1];\n    }\n";
+    h << "    return fl[(k == 0 ? HYX_XB : HYX_XB + HYX_NX + (k - 1) * HYX_RS) + t.vc[o]];\n}\n";
+
     Gen gen(gp.tmpl, P, high_acc);
     gen.split_min = split_min;
-    gen.literal_pow = false;
+    // Two waves per SIMD leave no registers for the i c^[i] history of the general pow form.
+    gen.literal_pow = derived;
+    gen.newest_last = derived;
+    if (derived) gen.find_sumsq(gp.outs);
+    gen.raw_inputs = derived && gen.inputs_only_linear();
+    // Two waves per SIMD where a lane's histories and the 66 registers that sums, addresses and
+    // scales get along with fit in 256 registers, and eight blocks in the 160 KB of LDS of a CU
+    // (six bodies at order 19: 49 registers spill, outside the recurrences, and the step
+    // takes 29 ms where it takes 36 ms at one wave per SIMD without spills; order 24 would
+    // spill histories).
+    const int hist = history_nodes(gp.tmpl) - (gen.raw_inputs ? nin : 0);
+    if (derived && !E && 2 * hist * (P - 1) + 66 <= 256 &&
+        (long)(flat + 16) * (64 / G) * 8 <= 20 * 1024)
+        h << "#define HYX_GROUP_WAVES 2\n";
     gen.perlane = gp.perlane;
     gen.kc_prefix = "tab.kc";
     auto &o = gen.o;
     auto xv = [](int oo, int k) { return "x" + std::to_string(oo) + "_" + std::to_string(k); };
-    auto X = [&](int k, const std::string &col) { return "fl[" + std::to_string(xb + k * nx) + " + " + col + "]"; };
+    auto X = [&](int k, const std::string &col) {
+        return "fl[" + std::to_string(k == 0 ? xb : xb + nx + (k - 1) * rs) + " + " + col + "]";
+    };
     auto vcol = [&](int oo) { return "vc" + std::to_string(oo); };
     o << "template <bool WTC, class TAB>\n"
          "__device__ __forceinline__ void hyx_gstep(double (&xo)[HYX_OWN], const double (&pv)[HYX_NPAR], double t0, "
-         "double max_dt, double &h_out, bool &nf_out, int g, double *fl, const TAB &tab, double *__restrict__ tc, "
+         "const double &max_dt, double &h_out, bool &nf_out, int g, double *fl, const TAB &tab, double *__restrict__ tc, "
          "hyx_u64 tcs"
       << (E ? ", unsigned long long &hyx_evm, double &hyx_mx" : "") << ")\n{\n";
     o << "    (void)pv; (void)t0; (void)tc; (void)tcs; (void)g;\n";
@@ -1775,7 +2076,9 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
     o << "    hyx_wsync();\n";
     // Owner sum of slot oo for x^[k+1], from the term values t_o (outputs) and t_s (state).
     auto owner_expr = [&](int oo, int k, const std::vector<std::string> &t_o, const std::vector<std::string> &t_s) {
-        std::string r = (k == 0) ? "tab.rc[" + std::to_string(oo) + "]" : "";
+        bool rc_nonzero = !derived;
+        for (int g = 0; g < G; ++g) rc_nonzero = rc_nonzero || gp.rc[(size_t)g * own + oo] != 0.0;
+        std::string r = (k == 0 && rc_nonzero) ? "tab.rc[" + std::to_string(oo) + "]" : "";
         auto add = [&](const std::string &sg, const std::string &val) {
             if (sg == "+")
                 r = r.empty() ? val : "(" + r + " + " + val + ")";
@@ -1812,13 +2115,16 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
         // the whole group, whose LDS accesses complete in issue order.
         o << "    // order 0\n";
         for (int q = 0; q < nin; ++q)
-            o << "    const double " << Gen::cv((uint32_t)q, 0) << " = " << X(0, "tab.iv[" + std::to_string(q) + "]") << ";\n";
+            o << "    const double " << Gen::cv((uint32_t)q, 0) << " = "
+              << (derived ? "fl[" + std::to_string(xb + rs) + " + tab.lis[" + std::to_string(q) + "]]"
+                          : X(0, "tab.iv[" + std::to_string(q) + "]"))
+              << ";\n";
         cluster_order(0);
         o << "    hyx_wsync();\n";
         for (int k = 1; k <= P; ++k) {
             o << "    // owner loads of order " << k - 1 << (k < P ? ", cluster order " + std::to_string(k) : "") << "\n";
             std::vector<std::vector<std::string>> to(own), ts(own);
-            for (int oo = 0; oo < own; ++oo) {
+            for (int oo = 0; oo < own_a; ++oo) {
                 for (int t = 0; t < gp.nto[oo]; ++t) {
                     const std::string nm = "ot" + std::to_string(oo) + "_" + std::to_string(t) + "_" + std::to_string(k);
                     o << "    const double " << nm << " = fl[tab.tio" << oo << "[" << t << "]];\n";
@@ -1846,11 +2152,16 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
                             r = r.empty() ? "(" + sgv + " * " + val + ")" : "__builtin_fma(" + sgv + ", " + val + ", " + r + ")";
                     }
                     if (r.empty()) r = "0.0";
-                    o << "    const double " << Gen::cv((uint32_t)q, k) << " = " << r << " * " << lit(1.0 / k) << ";\n";
+                    o << "    const double " << Gen::cv((uint32_t)q, k) << " = " << r
+                      << (gen.raw_inputs ? "" : " * " + lit(1.0 / k)) << ";\n";
                 }
+            // Sums that the exchange under way does not enter, while it is.
+            if (k < P)
+                for (uint32_t j = gp.tmpl.n; j < gp.tmpl.nnodes; ++j) gen.pre_order(j, k);
             // The owners finish order k before the cluster work, so no sum stays live across it.
-            for (int oo = 0; oo < own; ++oo) {
-                o << "    const double " << xv(oo, k) << " = " << owner_expr(oo, k - 1, to[oo], ts[oo]) << ";\n";
+            for (int oo = 0; oo < own_a; ++oo) {
+                const std::string sum = owner_expr(oo, k - 1, to[oo], ts[oo]);
+                o << "    const double " << xv(oo, k) << " = " << sum << ";\n";
                 o << "    " << X(k, vcol(oo)) << " = " << xv(oo, k) << ";\n";
             }
             if (k < P) {
@@ -1881,16 +2192,18 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
     for (int oo = 0; oo < own; ++oo) {
         o << "        if (tab.vo[" << oo << "] >= 0)\n";
         o << "            for (int k = 0; k <= HYX_P; ++k) tc[((hyx_u64)tab.vo[" << oo << "] * " << (P + 1)
-          << " + k) * tcs] = fl[HYX_XB + k * HYX_NX + " << vcol(oo) << "];\n";
+          << " + k) * tcs] = hyx_grow(fl, tab, " << oo << ", k);\n";
     }
     o << "    }\n";
     if (E) {
         // Event functions: every lane of the group forms the whole jet from the state
         // rows in LDS (broadcast reads), so the group agrees without an exchange.
         Gen eg(*E, P, high_acc);
-        eg.lds_xb = xb;
-        eg.lds_nx = nx;
-        eg.lds_col = col;
+        eg.lds_row = [&](uint32_t i, int k) {
+            const int v = gp.dsrc[i];
+            if (v < 0 || k == 0) return X(k, std::to_string(col[i]));
+            return "(" + X(k - 1, std::to_string(col[(size_t)v])) + " * " + lit(1.0 / k) + ")";
+        };
         o << "    double hyx_evg[" << nev << "][" << (P + 1) << "];\n    {\n";
         for (uint32_t j = E->n; j < E->nnodes; ++j) eg.order0(j);
         for (int k = 1; k <= P; ++k)
@@ -1903,18 +2216,21 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
     }
     o << "    double mx = 0.0, mo = 0.0, mom1 = 0.0;\n";
     for (int oo = 0; oo < own; ++oo) {
-        o << "    mx = fmax(mx, fabs(" << xv(oo, 0) << "));\n";
-        o << "    mo = fmax(mo, fabs(" << xv(oo, P) << "));\n";
-        o << "    mom1 = fmax(mom1, fabs(" << xv(oo, P - 1) << "));\n";
+        // The orders 0, p and p - 1 of a slot (derived mode: order 0 is read back, so that it
+        // is not held in registers through the step).
+        const bool d = oo >= own_a;
+        const std::string x0 = derived ? X(0, vcol(oo)) : xv(oo, 0);
+        const std::string xp = d ? xv(oo - own_a, P - 1) + " * " + lit(1.0 / P) : xv(oo, P);
+        const std::string xq = d ? xv(oo - own_a, P - 2) + " * " + lit(1.0 / (P - 1)) : xv(oo, P - 1);
+        o << "    mx = fmax(mx, fabs(" << x0 << "));\n";
+        o << "    mo = fmax(mo, fabs(" << xp << "));\n";
+        o << "    mom1 = fmax(mom1, fabs(" << xq << "));\n";
     }
     for (uint32_t e = 0; E && e < nev; ++e) {
         o << "    mo = fmax(mo, fabs(hyx_evg[" << e << "][" << P << "]));\n";
         o << "    mom1 = fmax(mom1, fabs(hyx_evg[" << e << "][" << (P - 1) << "]));\n";
     }
-    o << "#pragma unroll\n    for (int off = 1; off < HYX_G; off <<= 1) {\n"
-         "        mx = fmax(mx, __shfl_xor(mx, off));\n"
-         "        mo = fmax(mo, __shfl_xor(mo, off));\n"
-         "        mom1 = fmax(mom1, __shfl_xor(mom1, off));\n    }\n";
+    group_norms(o, G);
     step_size(o, P);
     if (E) {
         // The same fast exclusion as the lane forms; the coefficients of the steps it
@@ -1940,27 +2256,39 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
         for (int oo = 0; oo < own; ++oo) {
             o << "            if (tab.vo[" << oo << "] >= 0)\n";
             o << "                for (int k = 0; k <= HYX_P; ++k) tc[((hyx_u64)tab.vo[" << oo << "] * " << (P + 1)
-              << " + k) * tcs] = fl[HYX_XB + k * HYX_NX + " << vcol(oo) << "];\n";
+              << " + k) * tcs] = hyx_grow(fl, tab, " << oo << ", k);\n";
         }
         o << "        }\n    }\n";
         o << "    hyx_mx = mx;\n";
     }
     o << "    int nf = 0;\n";
     // State update from the coefficient rows in LDS.
-    for (int oo = 0; oo < own; ++oo) {
-        if (!high_acc) {
+    for (int oo = 0; oo < own_a; ++oo) {
+        const int d = oo + own_a;
+        if (!high_acc && derived) {
+            // The variable and the one derived from it, in one pass over the rows.
+            o << "    { double c = " << X(P - 1, vcol(oo)) << ", r = __builtin_fma(" << xv(oo, P) << ", h, c), s = c * "
+              << lit(1.0 / P) << ";\n";
+            for (int k = P - 1; k >= 1; --k)
+                o << "      c = " << X(k - 1, vcol(oo)) << "; r = __builtin_fma(r, h, c); s = __builtin_fma(s, h, c * "
+                  << lit(1.0 / k) << ");\n";
+            o << "      s = __builtin_fma(s, h, " << X(0, vcol(d)) << ");\n";
+            o << "      xo[" << oo << "] = r; xo[" << d << "] = s; nf |= (isfinite(r) && isfinite(s)) ? 0 : 1; }\n";
+        } else if (!high_acc) {
             o << "    { double r = " << xv(oo, P) << ";\n";
-            o << "#pragma unroll\n      for (int k = HYX_P - 1; k >= 0; --k) r = __builtin_fma(r, h, fl[HYX_XB + k * HYX_NX + "
-              << vcol(oo) << "]);\n";
-        } else {
-            o << "    { double r = " << xv(oo, 0) << ", cp = 0.0, hk = 1.0;\n";
-            o << "#pragma unroll\n      for (int k = 1; k <= HYX_P; ++k) { hk *= h; const double y = fl[HYX_XB + k * HYX_NX + "
-              << vcol(oo) << "] * hk - cp; const double tt = r + y; cp = (tt - r) - y; r = tt; }\n";
+            for (int k = P - 1; k >= 0; --k) o << "      r = __builtin_fma(r, h, " << X(k, vcol(oo)) << ");\n";
+            o << "      xo[" << oo << "] = r; nf |= (tab.vo[" << oo << "] >= 0 && !isfinite(r)) ? 1 : 0; }\n";
         }
+    }
+    for (int oo = 0; high_acc && oo < own; ++oo) {
+        o << "    { double r = " << X(0, vcol(oo)) << ", cp = 0.0, hk = 1.0;\n";
+        for (int k = 1; k <= P; ++k)
+            o << "      { hk *= h; const double y = "
+              << (oo < own_a ? X(k, vcol(oo)) : "(" + X(k - 1, vcol(oo - own_a)) + " * " + lit(1.0 / k) + ")")
+              << " * hk - cp; const double tt = r + y; cp = (tt - r) - y; r = tt; }\n";
         o << "      xo[" << oo << "] = r; nf |= (tab.vo[" << oo << "] >= 0 && !isfinite(r)) ? 1 : 0; }\n";
     }
-    o << "#pragma unroll\n    for (int off = 1; off < HYX_G; off <<= 1) nf |= __shfl_xor(nf, off);\n";
-    o << "    h_out = h;\n    nf_out = nf != 0;\n}\n";
+    o << "    nf_out = hyx_gany(nf) != 0;\n    h_out = h;\n}\n";
     return h.str() + o.str();
 }
 
@@ -3178,7 +3506,8 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
     h << "#define HYX_N " << n << "\n#define HYX_NPAR " << std::max<uint32_t>(S.npar, 1) << "\n#define HYX_P " << P
       << "\n#define HYX_GROUP 1\n#define HYX_WAVE 1\n#define HYX_G " << G << "\n#define HYX_I " << ipb
       << "\n#define HYX_OWN " << own << "\n#define HYX_NX " << R << "\n#define HYX_XB 0\n#define HYX_FLAT " << flat
-      << "\n#define HYX_WAVE_SLOTS " << slots.size() << "\n";
+      << "\n#define HYX_WAVE_SLOTS " << slots.size() << "\n#define HYX_VO(o) hyx_wtab_vo[g * HYX_OWN + (o)]\n";
+    if ((long)(flat + 14) * ipb * 8 > 160 * 1024) h << "#define HYX_REC_REGS 1\n";
     h << "typedef unsigned long long hyx_u64;\n";
     h << "#ifndef HYX_CPU_EMU\n"
          "// A block is one wavefront, and the LDS operations of a wavefront complete in issue\n"
@@ -3189,6 +3518,7 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
          "    __builtin_amdgcn_wave_barrier();\n"
          "    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");\n}\n"
          "#endif\n";
+    h << group_fold_src();
 
     // Slot code. Operand rows are per-lane registers tab.w[f]; T[k][row] is fl[row + k * R].
     auto Tk = [&](const std::string &row, int k) {
@@ -3603,11 +3933,14 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
     if (!D.empty()) h << "    for (int f = 0; f < " << D.size() << "; ++f) t.d[f] = hyx_wtab_d[f * HYX_G + g];\n";
     h << "}\n";
 
+    h << "__device__ __forceinline__ double hyx_grow(const double *fl, const hyx_gtab &t, int o, int k)\n{\n"
+         "    return fl[HYX_XB + k * HYX_NX + t.vc[o]];\n}\n";
+
     auto xv = [](int oo, int k) { return "x" + std::to_string(oo) + "_" + std::to_string(k); };
     auto vcol = [](int oo) { return "vc" + std::to_string(oo); };
     o << "template <bool WTC, class TAB>\n"
          "__device__ __forceinline__ void hyx_gstep(double (&xo)[HYX_OWN], const double (&pv)[HYX_NPAR], double t0, "
-         "double max_dt, double &h_out, bool &nf_out, int g, double *fl, const TAB &tab, double *__restrict__ tc, "
+         "const double &max_dt, double &h_out, bool &nf_out, int g, double *fl, const TAB &tab, double *__restrict__ tc, "
          "hyx_u64 tcs"
       << (E ? ", unsigned long long &hyx_evm, double &hyx_mx" : "") << ")\n{\n";
     o << "    (void)pv; (void)t0; (void)tc; (void)tcs; (void)g;\n";
@@ -3671,8 +4004,7 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
     o << "    }\n";
     if (E) {
         Gen eg(*E, P, high_acc);
-        eg.lds_xb = 0;
-        eg.lds_nx = R;
+        eg.lds_row = [&](uint32_t i, int k) { return "fl[" + std::to_string(k * R + (int)i) + "]"; };
         o << "    double hyx_evg[" << nev << "][" << (P + 1) << "];\n    {\n";
         for (uint32_t j = E->n; j < E->nnodes; ++j) eg.order0(j);
         for (int k = 1; k <= P; ++k)
@@ -3693,10 +4025,7 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
         o << "    mo = fmax(mo, fabs(hyx_evg[" << e << "][" << P << "]));\n";
         o << "    mom1 = fmax(mom1, fabs(hyx_evg[" << e << "][" << (P - 1) << "]));\n";
     }
-    o << "#pragma unroll\n    for (int off = 1; off < HYX_G; off <<= 1) {\n"
-         "        mx = fmax(mx, __shfl_xor(mx, off));\n"
-         "        mo = fmax(mo, __shfl_xor(mo, off));\n"
-         "        mom1 = fmax(mom1, __shfl_xor(mom1, off));\n    }\n";
+    group_norms(o, G);
     step_size(o, P);
     if (E) {
         const uint64_t off = (uint64_t)n * (P + 1) + (uint64_t)(E->nnodes - E->n) * (P + 1);
@@ -3737,8 +4066,7 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
         }
         o << "      xo[" << oo << "] = r; nf |= (tab.vo[" << oo << "] >= 0 && !isfinite(r)) ? 1 : 0; }\n";
     }
-    o << "#pragma unroll\n    for (int off = 1; off < HYX_G; off <<= 1) nf |= __shfl_xor(nf, off);\n";
-    o << "    h_out = h;\n    nf_out = nf != 0;\n}\n";
+    o << "    nf_out = hyx_gany(nf) != 0;\n    h_out = h;\n}\n";
     return h.str() + o.str();
 }
 

@@ -86,18 +86,24 @@ struct GroupPlan {
     std::vector<int> iv;            // [G][nin] state variable of each input
     std::vector<double> kc;         // [G][nkc] constants
     // Owned state variables: lane g, slot o owns vo[g][o] (-1: none). Its right-hand
-    // side is rc + sum of output terms (LDS output index, sign) + sum of state terms
-    // (variable index, sign); per slot, nto[o] / nts[o] terms (padded: output index
+    // side is rc + sum of output terms (LDS output index, scale) + sum of state terms
+    // (variable index, scale); per slot, nto[o] / nts[o] terms (padded: output index
     // os * nout and variable index n read zeros).
     std::vector<int> vo;            // [G][own]
     std::vector<double> rc;         // [G][own]
     std::vector<int> nto, nts;      // [own]
     std::vector<std::vector<int>> tio, tis;          // [own][G * nto[o]] / [own][G * nts[o]]
-    std::vector<std::vector<double>> tso, tss;       // signs, same shapes
+    std::vector<std::vector<double>> tso, tss;       // scales, same shapes
+    // Derived variables (own_a < own): every cluster input is a variable x with x' = v (N-body
+    // positions), so x^[k] = v^[k-1] / k is formed where it is read and only x^[0] is
+    // stored. Slots 0 .. own_a - 1 own the other variables, slot own_a + o of a lane the one
+    // derived from its slot o's (if any).
+    int own_a = 0;
+    std::vector<int> dsrc;          // [n] the variable x is derived from, or -1
 };
 
-bool plan_groups(const Sys &S, GroupPlan &gp, std::string &why);
 // pipeline: one LDS exchange per order when every cluster input is a lagged state variable.
+bool plan_groups(const Sys &S, GroupPlan &gp, std::string &why, bool pipeline = true);
 // With events (E, nev) the step takes `unsigned long long &hyx_evm, double &hyx_mx`
 // (per-event root-scan flags, and the group's max |x| at the start of the step).
 std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int order, bool high_acc, int split_min = 0,

@@ -31,17 +31,40 @@
 // the group then runs the detection of hyx_kevent.hip (every lane the same) and,
 // at a terminal trigger, re-evaluates its owned variables from the LDS rows.
 
+//
+// What a step neither reads nor changes (the propagation's bookkeeping, the same for every
+// lane of the group) waits in LDS, one record per group: hyx_gstep's fences make the
+// compiler read it back after the step, instead of holding some 30 registers per lane
+// through it. With HYX_GROUP_WAVES the kernels keep to the 256 registers of two
+// wavefronts per SIMD: a SIMD issues from one wave while the other waits for its LDS
+// exchange or issues scalar and LDS instructions. 65,536 six-body systems to t = 10, kernel:
+// 48.3 ms with six outputs per pair, position rows and bookkeeping in registers (one wave
+// per SIMD: 382 registers, 28 KB of LDS); 36.5 ms with this layout at one wave, 28.7 ms at two
+// (VALU busy 72 % of the cycles, 2,000 VALU of 2,660 instructions per wave-step).
+struct hyx_grec {
+    double thi, tlo, tfhi, tflo, mdt, minh, maxh;
+    double hlast; // the last step's size (kept for the host when the instance parks)
+    double rem, lim; // remaining time and step limit of the running step
+    hyx_u64 iter, nst;
+    hyx_u64 inst, budget; // persistent kernel: the instance and its iterations in this launch
+};
+
+#ifdef HYX_GROUP_WAVES
+#define HYX_GROUP_ATTR __attribute__((amdgpu_waves_per_eu(HYX_GROUP_WAVES, HYX_GROUP_WAVES)))
+#else
+#define HYX_GROUP_ATTR
+#endif
+
 struct hyx_ginst {
     double xo[HYX_OWN];
     double pv[HYX_NPAR];
-    double thi, tlo, tfhi, tflo, mdt, minh, maxh;
-    hyx_u64 iter, nst;
-    double hlast; // the last step's size (kept for the host when the instance parks)
     int tdir;
     unsigned gc; // propagate_grid: next grid point
 #ifdef HYX_EVENTS
     unsigned long long cdact; // terminal events with a running cooldown
 #endif
+    hyx_grec &r;
+    __device__ __forceinline__ hyx_ginst(hyx_grec &rec) : r(rec) {}
 };
 
 #ifdef HYX_EVENTS
@@ -60,19 +83,18 @@ __device__ __forceinline__ double hyx_gevents(hyx_ginst &s, const hyx_kargs &a, 
 #pragma unroll
     for (int o = 0; o < HYX_OWN; ++o) {
         if (t.vo[o] < 0) continue;
-        const double *row = fl + HYX_XB + t.vc[o];
 #ifdef HYX_HIGH_ACC
-        double r = row[0], cp = 0.0, hk = 1.0;
+        double r = hyx_grow(fl, t, o, 0), cp = 0.0, hk = 1.0;
         for (int k = 1; k <= HYX_P; ++k) {
             hk *= hend;
-            const double y = row[k * HYX_NX] * hk - cp;
+            const double y = hyx_grow(fl, t, o, k) * hk - cp;
             const double tt = r + y;
             cp = (tt - r) - y;
             r = tt;
         }
 #else
-        double r = row[HYX_P * HYX_NX];
-        for (int k = HYX_P - 1; k >= 0; --k) r = __builtin_fma(r, hend, row[k * HYX_NX]);
+        double r = hyx_grow(fl, t, o, HYX_P);
+        for (int k = HYX_P - 1; k >= 0; --k) r = __builtin_fma(r, hend, hyx_grow(fl, t, o, k));
 #endif
         s.xo[o] = r;
         bad |= isfinite(r) ? 0 : 1;
@@ -88,11 +110,11 @@ __device__ __forceinline__ void hyx_gload(hyx_ginst &s, const hyx_kargs &a, hyx_
 {
 #pragma unroll
     for (int o = 0; o < HYX_OWN; ++o)
-        s.xo[o] = (t.vo[o] >= 0) ? a.state[(hyx_u64)t.vo[o] * a.ld + i] : 0.0;
+        s.xo[o] = (HYX_VO(o) >= 0) ? a.state[(hyx_u64)HYX_VO(o) * a.ld + i] : 0.0;
 #pragma unroll
     for (int q = 0; q < HYX_NPAR; ++q) s.pv[q] = a.pars ? a.pars[(hyx_u64)q * a.ld + i] : 0.0;
-    s.thi = a.t_hi[i];
-    s.tlo = a.t_lo[i];
+    s.r.thi = a.t_hi[i];
+    s.r.tlo = a.t_lo[i];
 }
 
 __device__ __forceinline__ void hyx_gstore_state(const hyx_ginst &s, const hyx_kargs &a, hyx_u64 i, int g,
@@ -100,10 +122,10 @@ __device__ __forceinline__ void hyx_gstore_state(const hyx_ginst &s, const hyx_k
 {
 #pragma unroll
     for (int o = 0; o < HYX_OWN; ++o)
-        if (t.vo[o] >= 0) a.state[(hyx_u64)t.vo[o] * a.ld + i] = s.xo[o];
+        if (HYX_VO(o) >= 0) a.state[(hyx_u64)HYX_VO(o) * a.ld + i] = s.xo[o];
     if (g == 0) {
-        a.t_hi[i] = s.thi;
-        a.t_lo[i] = s.tlo;
+        a.t_hi[i] = s.r.thi;
+        a.t_lo[i] = s.r.tlo;
     }
 }
 
@@ -111,14 +133,14 @@ __device__ __forceinline__ void hyx_gresume(hyx_ginst &s, const hyx_kargs &a, hy
                                             const hyx_gtab &t)
 {
     hyx_gload(s, a, i, g, t);
-    s.tfhi = a.tf_hi[i];
-    s.tflo = a.tf_lo[i];
-    s.mdt = a.max_dt[i];
+    s.r.tfhi = a.tf_hi[i];
+    s.r.tflo = a.tf_lo[i];
+    s.r.mdt = a.max_dt[i];
     s.tdir = (st == 0u);
-    s.minh = a.min_h[i];
-    s.maxh = a.max_h[i];
-    s.iter = a.iters[i];
-    s.nst = a.nsteps[i];
+    s.r.minh = a.min_h[i];
+    s.r.maxh = a.max_h[i];
+    s.r.iter = a.iters[i];
+    s.r.nst = a.nsteps[i];
 #ifdef HYX_GRID
     s.gc = a.gcur[i];
 #endif
@@ -132,16 +154,16 @@ __device__ __forceinline__ void hyx_gsuspend(const hyx_ginst &s, const hyx_kargs
 {
     hyx_gstore_state(s, a, i, g, t);
     if (g == 0) {
-        a.min_h[i] = s.minh;
-        a.max_h[i] = s.maxh;
-        a.iters[i] = s.iter;
-        a.nsteps[i] = s.nst;
+        a.min_h[i] = s.r.minh;
+        a.max_h[i] = s.r.maxh;
+        a.iters[i] = s.r.iter;
+        a.nsteps[i] = s.r.nst;
 #ifdef HYX_GRID
         a.gcur[i] = s.gc;
 #endif
         if (done && res == HYX_PARKED) {
             a.status[i] = HYX_ST_PARKED | (s.tdir ? 0u : 2u);
-            a.h_out[i] = s.hlast;
+            a.h_out[i] = s.r.hlast;
         } else if (done) {
             a.status[i] = HYX_ST_DONE;
             a.outcome[i] = res;
@@ -160,14 +182,13 @@ __device__ __forceinline__ void hyx_ggrid(hyx_ginst &s, const hyx_kargs &a, hyx_
     unsigned c = s.gc;
     while (c < a.npts) {
         bool inside;
-        const double dt = hyx_grid_offset(a.grid[(hyx_u64)c * a.ld + i], s.thi, s.tlo, h, s.tdir, inside);
+        const double dt = hyx_grid_offset(a.grid[(hyx_u64)c * a.ld + i], s.r.thi, s.r.tlo, h, s.tdir, inside);
         if (!inside && !fin) break;
 #pragma unroll
         for (int o = 0; o < HYX_OWN; ++o) {
             if (t.vo[o] < 0) continue;
-            const double *row = fl + HYX_XB + t.vc[o];
-            double r = row[HYX_P * HYX_NX];
-            for (int k = HYX_P - 1; k >= 0; --k) r = __builtin_fma(r, dt, row[k * HYX_NX]);
+            double r = hyx_grow(fl, t, o, HYX_P);
+            for (int k = HYX_P - 1; k >= 0; --k) r = __builtin_fma(r, dt, hyx_grow(fl, t, o, k));
             a.gout[((hyx_u64)c * HYX_N + t.vo[o]) * a.ld + i] = r;
         }
         ++c;
@@ -185,8 +206,9 @@ __device__ __forceinline__ bool hyx_gprop_iter(hyx_ginst &s, const hyx_kargs &a,
 {
     (void)i;
     (void)wr;
-    const double rem = hyx_dfl_sub_hi(s.tfhi, s.tflo, s.thi, s.tlo);
-    const double lim = s.tdir ? ((s.mdt < rem) ? s.mdt : rem) : ((-s.mdt > rem) ? -s.mdt : rem);
+    hyx_grec &r = s.r;
+    r.rem = hyx_dfl_sub_hi(r.tfhi, r.tflo, r.thi, r.tlo);
+    r.lim = s.tdir ? ((r.mdt < r.rem) ? r.mdt : r.rem) : ((-r.mdt > r.rem) ? -r.mdt : r.rem);
     double h;
     bool nf;
     int te = -1;
@@ -194,27 +216,32 @@ __device__ __forceinline__ bool hyx_gprop_iter(hyx_ginst &s, const hyx_kargs &a,
 #ifdef HYX_EVENTS
     unsigned long long evm = 0;
     double gmx = 0.0;
-    hyx_gstep<false>(s.xo, s.pv, s.thi, lim, h, nf, g, fl, t, wr ? a.tc + i : nullptr, a.ld, evm, gmx);
+    hyx_gstep<false>(s.xo, s.pv, r.thi, r.lim, h, nf, g, fl, t, wr ? a.tc + i : nullptr, a.ld, evm, gmx);
     if (wr) {
         unsigned ntc = 0;
-        h = hyx_gevents(s, a, i, fl, t, s.thi, s.tlo, h, evm, gmx, nf, te, ntc, false);
+        h = hyx_gevents(s, a, i, fl, t, r.thi, r.tlo, h, evm, gmx, nf, te, ntc, false);
         park = a.ev_pause && ((te >= 0 && !hyx_ev_stop[te]) || ntc > 0u);
     }
 #else
-    hyx_gstep<false>(s.xo, s.pv, s.thi, lim, h, nf, g, fl, t, nullptr, 0);
+    hyx_gstep<false>(s.xo, s.pv, r.thi, r.lim, h, nf, g, fl, t, nullptr, 0);
 #endif
-    hyx_dfl_add(s.thi, s.tlo, h, 0.0);
-    s.hlast = h;
-    nf = nf || !isfinite(s.thi);
-    s.iter += 1;
-    s.nst += (h != 0.0) ? 1 : 0;
-    const hyx_i64 oc = nf ? HYX_ERR_NF_STATE : ((te < 0 && h == lim) ? HYX_TIME_LIMIT : HYX_SUCCESS);
+    double thi = r.thi, tlo = r.tlo;
+    hyx_dfl_add(thi, tlo, h, 0.0);
+    r.thi = thi;
+    r.tlo = tlo;
+    r.hlast = h;
+    nf = nf || !isfinite(thi);
+    const hyx_u64 iter = r.iter + 1;
+    r.iter = iter;
+    if (h != 0.0) r.nst += 1;
+    const double rem = r.rem;
+    const hyx_i64 oc = nf ? HYX_ERR_NF_STATE : ((te < 0 && h == r.lim) ? HYX_TIME_LIMIT : HYX_SUCCESS);
     // min_h / max_h over steps the rule chose alone: not those clamped by the time limit
     // or shortened by a terminal event.
     if (oc == HYX_SUCCESS && te < 0) {
         const double ah = fabs(h);
-        s.minh = (ah < s.minh) ? ah : s.minh;
-        s.maxh = (ah > s.maxh) ? ah : s.maxh;
+        r.minh = (ah < r.minh) ? ah : r.minh;
+        r.maxh = (ah > r.maxh) ? ah : r.maxh;
     }
     if (oc == HYX_ERR_NF_STATE) {
         *res = HYX_ERR_NF_STATE;
@@ -236,7 +263,7 @@ __device__ __forceinline__ bool hyx_gprop_iter(hyx_ginst &s, const hyx_kargs &a,
         *res = HYX_TIME_LIMIT;
         return true;
     }
-    if (a.max_steps != 0 && s.iter >= a.max_steps) {
+    if (a.max_steps != 0 && iter >= a.max_steps) {
         *res = HYX_STEP_LIMIT;
         return true;
     }
@@ -245,6 +272,7 @@ __device__ __forceinline__ bool hyx_gprop_iter(hyx_ginst &s, const hyx_kargs &a,
 
 #define HYX_GROUP_SETUP                                                                                               \
     __shared__ double hyx_lds[HYX_I][HYX_FLAT];                                                                      \
+    HYX_GROUP_REC                                                                                                    \
     const int lane = (int)__lane_id();                                                                               \
     const int grp = lane / HYX_G;                                                                                    \
     const int g = lane % HYX_G;                                                                                      \
@@ -252,7 +280,18 @@ __device__ __forceinline__ bool hyx_gprop_iter(hyx_ginst &s, const hyx_kargs &a,
     for (int q = g; q < HYX_FLAT; q += HYX_G) fl[q] = 0.0;                                                           \
     hyx_gtab tab;                                                                                                    \
     hyx_gtab_load(tab, g);                                                                                           \
+    HYX_GROUP_INST                                                                                                   \
     hyx_wsync();
+
+// The groups' records; a wave form whose rows leave no room for them in the 160 KB of LDS
+// keeps them in registers.
+#ifdef HYX_REC_REGS
+#define HYX_GROUP_REC hyx_grec hyx_rec;
+#define HYX_GROUP_INST hyx_ginst s(hyx_rec);
+#else
+#define HYX_GROUP_REC __shared__ hyx_grec hyx_rec[HYX_I];
+#define HYX_GROUP_INST hyx_ginst s(hyx_rec[grp]);
+#endif
 
 // ---- step(): one adaptive step per instance ----------------------------------------------
 template <bool WTC>
@@ -262,7 +301,6 @@ __device__ __forceinline__ void hyx_gstep_body(const hyx_kargs &a)
     const hyx_u64 i = (hyx_u64)blockIdx.x * HYX_I + grp;
     const bool valid = i < a.N;
     const hyx_u64 ii = valid ? i : 0; // groups past the end step instance 0 and store nothing
-    hyx_ginst s;
     hyx_gload(s, a, ii, g, tab);
     const double mdt = a.max_dt[ii];
     double h;
@@ -271,17 +309,20 @@ __device__ __forceinline__ void hyx_gstep_body(const hyx_kargs &a)
 #ifdef HYX_EVENTS
     unsigned long long evm = 0;
     double gmx = 0.0;
-    hyx_gstep<WTC>(s.xo, s.pv, s.thi, mdt, h, nf, g, fl, tab, valid ? a.tc + i : nullptr, a.ld, evm, gmx);
+    hyx_gstep<WTC>(s.xo, s.pv, s.r.thi, mdt, h, nf, g, fl, tab, valid ? a.tc + i : nullptr, a.ld, evm, gmx);
     if (valid) {
         unsigned ntc = 0;
         s.cdact = hyx_ev_cdmask(a, i);
-        h = hyx_gevents(s, a, i, fl, tab, s.thi, s.tlo, h, evm, gmx, nf, te, ntc, true);
+        h = hyx_gevents(s, a, i, fl, tab, s.r.thi, s.r.tlo, h, evm, gmx, nf, te, ntc, true);
     }
 #else
-    hyx_gstep<WTC>(s.xo, s.pv, s.thi, mdt, h, nf, g, fl, tab, (WTC && valid) ? a.tc + i : nullptr, a.ld);
+    hyx_gstep<WTC>(s.xo, s.pv, s.r.thi, mdt, h, nf, g, fl, tab, (WTC && valid) ? a.tc + i : nullptr, a.ld);
 #endif
-    hyx_dfl_add(s.thi, s.tlo, h, 0.0);
-    nf = nf || !isfinite(s.thi);
+    double thi = s.r.thi, tlo = s.r.tlo;
+    hyx_dfl_add(thi, tlo, h, 0.0);
+    s.r.thi = thi;
+    s.r.tlo = tlo;
+    nf = nf || !isfinite(thi);
     if (valid) {
         hyx_gstore_state(s, a, i, g, tab);
         if (g == 0) {
@@ -292,9 +333,9 @@ __device__ __forceinline__ void hyx_gstep_body(const hyx_kargs &a)
     }
 }
 
-extern "C" __global__ void __launch_bounds__(64) hyx_step_k(hyx_kargs a) { hyx_gstep_body<false>(a); }
+extern "C" __global__ void __launch_bounds__(64) HYX_GROUP_ATTR hyx_step_k(hyx_kargs a) { hyx_gstep_body<false>(a); }
 
-extern "C" __global__ void __launch_bounds__(64) hyx_step_tc_k(hyx_kargs a) { hyx_gstep_body<true>(a); }
+extern "C" __global__ void __launch_bounds__(64) HYX_GROUP_ATTR hyx_step_tc_k(hyx_kargs a) { hyx_gstep_body<true>(a); }
 
 // ---- plain form: one propagate iteration per launch ----------------------------------------
 extern "C" __global__ void __launch_bounds__(64) hyx_iter_init_k(hyx_kargs a)
@@ -310,14 +351,13 @@ extern "C" __global__ void __launch_bounds__(64) hyx_iter_init_k(hyx_kargs a)
     a.outcome[i] = HYX_TIME_LIMIT;
 }
 
-extern "C" __global__ void __launch_bounds__(64) hyx_iter_k(hyx_kargs a)
+extern "C" __global__ void __launch_bounds__(64) HYX_GROUP_ATTR hyx_iter_k(hyx_kargs a)
 {
     HYX_GROUP_SETUP
     const hyx_u64 i = (hyx_u64)blockIdx.x * HYX_I + grp;
     const unsigned st = (i < a.N) ? a.status[i] : 1u;
     const bool valid = hyx_runnable(st);
     const hyx_u64 ii = (i < a.N) ? i : 0;
-    hyx_ginst s;
     hyx_gresume(s, a, ii, st, g, tab);
     hyx_i64 res = HYX_TIME_LIMIT;
     const bool done = hyx_gprop_iter(s, a, g, fl, tab, ii, valid, &res);
@@ -345,25 +385,16 @@ extern "C" __global__ void hyx_clear_u64_k(hyx_u64 *p, unsigned n)
 // this launch is written back unfinished (counted in *unfinished) and the host
 // launches again, so every wave leaves the loop after a bounded number of
 // iterations once the queue is drained.
-extern "C" __global__ void __launch_bounds__(64) hyx_persist_k(hyx_kargs a)
+extern "C" __global__ void __launch_bounds__(64) HYX_GROUP_ATTR hyx_persist_k(hyx_kargs a)
 {
     HYX_GROUP_SETUP
-    hyx_ginst s;
     hyx_gload(s, a, 0, g, tab);
-    s.tfhi = s.thi;
-    s.tflo = s.tlo;
-    s.mdt = 0.0;
+    s.r = hyx_grec{s.r.thi, s.r.tlo, s.r.thi, s.r.tlo, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0, 0, 0, 0};
     s.tdir = 1;
-    s.minh = 0.0;
-    s.maxh = 0.0;
-    s.iter = 0;
-    s.nst = 0;
-    s.hlast = 0.0;
     s.gc = 0;
 #ifdef HYX_EVENTS
     s.cdact = 0ull;
 #endif
-    hyx_u64 inst = 0, budget = 0;
     bool active = false;
     bool exhausted = false;
     for (;;) {
@@ -381,11 +412,12 @@ extern "C" __global__ void __launch_bounds__(64) hyx_persist_k(hyx_kargs a)
                 const hyx_u64 below_lead = (lead_lane == 0) ? 0ull : ((~0ull) >> (64 - lead_lane));
                 const hyx_u64 gpos = base + (hyx_u64)__popcll(idle & below_lead);
                 if (gpos < a.N) {
-                    inst = a.queue ? (hyx_u64)a.queue[gpos] : gpos;
+                    const hyx_u64 inst = a.queue ? (hyx_u64)a.queue[gpos] : gpos;
                     const unsigned st = a.status[inst];
                     if (hyx_runnable(st)) {
                         hyx_gresume(s, a, inst, st, g, tab);
-                        budget = 0;
+                        s.r.inst = inst;
+                        s.r.budget = 0;
                         active = true;
                     }
                 }
@@ -407,11 +439,12 @@ extern "C" __global__ void __launch_bounds__(64) hyx_persist_k(hyx_kargs a)
             for (;;) {
                 bool ended = false;
                 hyx_i64 res = HYX_TIME_LIMIT;
-                const bool done = hyx_gprop_iter(s, a, g, fl, tab, inst, active, &res);
+                const bool done = hyx_gprop_iter(s, a, g, fl, tab, s.r.inst, active, &res);
                 if (active) {
-                    budget += 1;
+                    const hyx_u64 budget = s.r.budget + 1;
+                    s.r.budget = budget;
                     if (done || budget >= a.iter_budget) {
-                        hyx_gsuspend(s, a, inst, g, tab, done, res);
+                        hyx_gsuspend(s, a, s.r.inst, g, tab, done, res);
                         if (!done && g == 0) atomicAdd(a.unfinished, 1u);
                         active = false;
                         ended = true;

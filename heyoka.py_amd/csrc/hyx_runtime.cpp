@@ -357,11 +357,11 @@ int build_sys(const uint32_t *ops, uint32_t n_words, const double *consts, uint3
         else if (flags & HYX_FLAG_FORCE_UNROLLED)
             s.form = HYX_FORM_UNROLLED;
         else if (flags & HYX_FLAG_FORCE_GROUP) {
-            if (!hyx::plan_groups(s.S, gp, why)) return fail(HYX_EINVAL, "the group form does not apply: " + why);
+            if (!hyx::plan_groups(s.S, gp, why, !(flags & HYX_FLAG_NO_PIPELINE))) return fail(HYX_EINVAL, "the group form does not apply: " + why);
             s.form = HYX_FORM_GROUP;
         } else if (flags & HYX_FLAG_FORCE_WAVE)
             s.form = HYX_FORM_WAVE;
-        else if (lane_compact && hyx::plan_groups(s.S, gp, why))
+        else if (lane_compact && hyx::plan_groups(s.S, gp, why, !(flags & HYX_FLAG_NO_PIPELINE)))
             s.form = HYX_FORM_GROUP;
         else
             s.form = lane_compact ? HYX_FORM_COMPACT : HYX_FORM_UNROLLED;
