@@ -846,11 +846,16 @@ struct Gen {
             o << "__device__ __forceinline__ double *hyx_xs_lane() { return hyx_xs + threadIdx.x; }\n";
             o << "#endif\n";
         }
-        o << "template <bool WTC>\n"
+        // propagate_grid's kernels evaluate the grid points of the step inside it, from the
+        // coefficients in registers (hyx_dense in hyx_klane.hip). With events the step may yet be
+        // shortened: there they evaluate from the coefficients in memory afterwards.
+        if (!E) o << "#ifdef HYX_GRID\n#define HYX_DENSE 1\n#define HYX_DENSE_ARG , DN &dn\n"
+                     "#define HYX_DENSE_TYPE , class DN\n#else\n#define HYX_DENSE_ARG\n#define HYX_DENSE_TYPE\n#endif\n";
+        o << "template <bool WTC" << (E ? "" : " HYX_DENSE_TYPE") << ">\n"
              "__device__ __forceinline__ void hyx_taylor_step(double (&x)[HYX_N], const double (&pv)[HYX_NPAR], "
              "double t0, double max_dt, double &h_out, bool &nf_out, double *__restrict__ tc, hyx_u64 tcs, "
              "double *__restrict__ tape, hyx_u64 tps"
-          << (E ? ", unsigned long long &hyx_evm" : "") << ")\n{\n";
+          << (E ? ", unsigned long long &hyx_evm" : " HYX_DENSE_ARG") << ")\n{\n";
         if (no_contract) o << "#pragma clang fp contract(off)\n";
         o << "    (void)pv; (void)t0; (void)tape; (void)tps; (void)tc; (void)tcs;\n";
         if (quad)
@@ -978,6 +983,15 @@ struct Gen {
                       << " * hk - cp; const double tt = sm + y; cp = (tt - sm) - y; sm = tt; }\n";
                 o << "      " << xo << "[" << i << "] = sm; nf = nf || !isfinite(sm); }\n";
             }
+        }
+        if (!E && !quad) {
+            o << "#ifdef HYX_DENSE\n    dn.begin(h, nf);\n    double dt;\n    while (dn.next(dt)) {\n";
+            for (uint32_t i = 0; i < n; ++i) {
+                o << "        { double r = " << nv(i, P) << ";\n";
+                for (int k = P - 1; k >= 0; --k) o << "          r = __builtin_fma(r, dt, " << nv(i, k) << ");\n";
+                o << "          dn.put(" << i << ", r); }\n";
+            }
+            o << "    }\n#endif\n";
         }
         if (quad)
             for (uint32_t i = 0; i < n; ++i)

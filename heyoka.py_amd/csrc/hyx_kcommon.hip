@@ -161,11 +161,23 @@ extern "C" __global__ void hyx_fill_u32_k(unsigned *p, unsigned v, hyx_u64 n)
     if (i < n) p[i] = v;
 }
 
-// Grid-stride fill of n 64-bit words (the NaN prefill of propagate_grid's output).
+// Grid-stride fill of n 64-bit words.
 extern "C" __global__ void hyx_fill_u64_k(hyx_u64 *p, hyx_u64 v, hyx_u64 n)
 {
     const hyx_u64 stride = (hyx_u64)gridDim.x * blockDim.x;
     for (hyx_u64 i = (hyx_u64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = v;
+}
+
+// propagate_grid's output at the points that instance i did not reach (from gcur[i] on): NaN,
+// [npts][n][ld]. After the propagation, so that the reached points are written once.
+extern "C" __global__ void hyx_grid_rest_k(double *out, const unsigned *gcur, hyx_u64 ld, unsigned n, hyx_u64 npts)
+{
+    const hyx_u64 stride = (hyx_u64)gridDim.x * blockDim.x;
+    for (hyx_u64 t = (hyx_u64)blockIdx.x * blockDim.x + threadIdx.x; t < npts * ld; t += stride) {
+        const hyx_u64 c = t / ld, i = t % ld;
+        if (c < gcur[i]) continue;
+        for (unsigned q = 0; q < n; ++q) out[(c * n + q) * ld + i] = __builtin_nan("");
+    }
 }
 
 // Dense-output time of grid point g for a step of size h that ended at

@@ -236,7 +236,7 @@ struct hyx_sys {
     // propagate_grid: the same source built with HYX_GRID, loaded on first use.
     std::mutex gmu;
     hipModule_t gmod = nullptr;
-    hipFunction_t kg_init = nullptr, kg_iter = nullptr, kg_persist = nullptr;
+    hipFunction_t kg_init = nullptr, kg_iter = nullptr, kg_persist = nullptr, kg_rest = nullptr;
     // Continuous output: the same source built with HYX_CLOG, loaded on first use.
     hipModule_t cmod = nullptr;
     hipFunction_t kc_init = nullptr, kc_iter = nullptr, kc_persist = nullptr;
@@ -1126,7 +1126,8 @@ int ensure_grid_module(hyx_sys *s)
     struct {
         hipFunction_t *f;
         const char *name;
-    } fns[] = {{&s->kg_init, "hyx_iter_init_k"}, {&s->kg_iter, "hyx_iter_k"}, {&s->kg_persist, "hyx_persist_k"}};
+    } fns[] = {{&s->kg_init, "hyx_iter_init_k"}, {&s->kg_iter, "hyx_iter_k"}, {&s->kg_persist, "hyx_persist_k"},
+               {&s->kg_rest, "hyx_grid_rest_k"}};
     for (auto &f : fns) {
         hipError_t e = hipModuleGetFunction(f.f, m, f.name);
         if (e != hipSuccess) {
@@ -1454,6 +1455,20 @@ int hyx_noalloc_propagate(hyx_sys *s, const hyx::NoAllocArgs &na, unsigned char 
 
 extern "C" {
 
+// The grid output so far, NaN at the points not reached (a propagation that ends early, as in
+// heyoka's batch propagate_grid).
+static int read_grid(hyx_batch *b, double *out)
+{
+    uint64_t npts = b->npts, N = b->N;
+    unsigned n = b->sys->S.n;
+    void *params[] = {&b->gout, &b->gcur, &N, &n, &npts};
+    const unsigned blocks = (unsigned)std::min<uint64_t>((npts * N + 255) / 256, 8192);
+    HIPCHK(hipModuleLaunchKernel(b->sys->kg_rest, blocks, 1, 1, 256, 1, 1, 0, b->stream, params, nullptr));
+    HIPCHK(hipMemcpyAsync(out, b->gout, npts * n * N * 8, hipMemcpyDeviceToHost, b->stream));
+    HIPCHK(hipStreamSynchronize(b->stream));
+    return 0;
+}
+
 int hyx_propagate_grid(hyx_batch *b, const double *grid, uint64_t n_pts, const double *max_delta_t,
                        uint64_t max_steps, int mode, hyx_prop_res *res, double *out)
 {
@@ -1482,18 +1497,12 @@ int hyx_propagate_grid(hyx_batch *b, const double *grid, uint64_t n_pts, const d
         }
     }
     if (int rc = ensure_grid_module(b->sys)) return rc;
-    if (!group_kernels(b->sys) && !b->tc) HIPCHK(hipMalloc((void **)&b->tc, (size_t)n * (P + 1) * N * 8));
+    if ((b->sys->compact || b->sys->has_events) && !b->tc) HIPCHK(hipMalloc((void **)&b->tc, (size_t)n * (P + 1) * N * 8));
     if (int rc = reserve(&b->grid, &b->grid_cap, n_pts * N)) return rc;
     if (int rc = reserve(&b->gout, &b->gout_cap, n_pts * n * N)) return rc;
     if (!b->gcur) HIPCHK(hipMalloc((void **)&b->gcur, N * 4));
     HIPCHK(hipMemcpyAsync(b->grid, grid, n_pts * N * 8, hipMemcpyHostToDevice, b->stream));
     {
-        // Unreached points stay NaN (a propagation that ends early, as in heyoka's batch propagate_grid).
-        uint64_t *p = (uint64_t *)b->gout;
-        uint64_t v = 0x7ff8000000000000ull, cnt = n_pts * n * N;
-        void *params[] = {&p, &v, &cnt};
-        const unsigned blocks = (unsigned)std::min<uint64_t>((cnt + 255) / 256, 8192);
-        HIPCHK(hipModuleLaunchKernel(b->sys->k_fill64, blocks, 1, 1, 256, 1, 1, 0, b->stream, params, nullptr));
         unsigned *q = b->gcur;
         unsigned one = 1;
         uint64_t nn = N;
@@ -1508,9 +1517,7 @@ int hyx_propagate_grid(hyx_batch *b, const double *grid, uint64_t n_pts, const d
     if (int rc = upload(b, b->mdt, max_delta_t, N, std::numeric_limits<double>::infinity())) return rc;
     b->npts = n_pts;
     if (int rc = run_propagation(b, max_steps, mode, res, true)) return rc;
-    HIPCHK(hipMemcpyAsync(out, b->gout, n_pts * n * N * 8, hipMemcpyDeviceToHost, b->stream));
-    HIPCHK(hipStreamSynchronize(b->stream));
-    return 0;
+    return read_grid(b, out);
 }
 
 int hyx_autotune(hyx_batch *b, const double *tf_hi, const char *cache_path, hyx_tune_res *best)
@@ -2034,8 +2041,7 @@ int hyx_propagate_resume(hyx_batch *b, uint64_t max_steps, int mode, hyx_prop_re
     const bool grid = b->last_grid;
     if (int rc = run_propagation(b, max_steps, mode, res, grid, false)) return rc;
     if (grid && grid_out) {
-        HIPCHK(hipMemcpyAsync(grid_out, b->gout, b->npts * b->sys->S.n * b->N * 8, hipMemcpyDeviceToHost, b->stream));
-        HIPCHK(hipStreamSynchronize(b->stream));
+        if (int rc = read_grid(b, grid_out)) return rc;
     }
     return 0;
 }
