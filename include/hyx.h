@@ -290,7 +290,8 @@ int hyx_autotune(hyx_batch *b, const double *tf_hi, const char *cache_path, hyx_
  * same arithmetic (HYX_FLAG_NO_QUAD: keep the twin). A persistent propagation hands its
  * last instances to it once its queue is drained and at most tail_min instances are in
  * flight (default: eight per CU; 0: never), so the longest-running instances of a ragged
- * ensemble take lower-latency steps. Results do not depend on the hand-off.
+ * ensemble take lower-latency steps; a batch of at most tail_min instances (by default: of at
+ * most 128 per CU) starts in it. Results do not depend on the hand-off.
  * hyx_sys_twin_source: that form's HIP source (length 0: the system has none);
  * hyx_batch_twin_launches: its launches in the batch's propagations so far. */
 int hyx_batch_set_twin_tail(hyx_batch *b, uint32_t tail_min);

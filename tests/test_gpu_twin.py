@@ -132,3 +132,19 @@ def test_quad_integrator_api_and_oracle():
                           lane_batch=1)
     err = np.max(np.abs(ta.state - r["state"]) / np.maximum(np.abs(r["state"]), 1.0))
     assert err < 1e-10, err
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 2049, 32768, 32769])
+def test_small_batches_start_in_the_tail_form(n):
+    # Batches up to 128 instances per CU start in the tail form (no lane-form launch before it);
+    # the same results as the plain lane form, bit for bit, on either side of the line.
+    print(f"[gpu] direct tail form n={n}", flush=True)
+    wl = W.cr3bp(n, log_t=(0.3, 1.0))
+    system = get_system(hy.taylor_decompose(wl.sys), 19)
+    ps, pt, pr, _ = _run(system, wl.state, wl.pars, wl.t_final, _lib.MODE_PLAIN)
+    qs, qt, qr, launches = _run(system, wl.state, wl.pars, wl.t_final, _lib.MODE_PERSISTENT)
+    assert launches > 0
+    done = pr["outcome"] == int(hy.taylor_outcome.time_limit)
+    assert done.mean() > 0.5 and np.array_equal(ps[:, done], qs[:, done]) and np.array_equal(pt, qt)
+    for k in ("outcome", "min_h", "max_h", "nsteps"):
+        assert np.array_equal(pr[k], qr[k]), k
