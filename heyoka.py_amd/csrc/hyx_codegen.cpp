@@ -227,9 +227,9 @@ struct Gen {
     bool lds_state = false;
     int cur_k = 0;
     // pow recurrence with literal coefficients (no i c^[i] history). Measured: the lane
-    // form's CR3BP step drops from 4,232 to 3,853 instructions and 411 to 341 registers;
-    // the group form's 6-body step runs 2.6 % slower with it (its register count stays
-    // above the two-wave threshold either way), so the group form keeps the other form.
+    // form's CR3BP step drops from 4,232 to 3,853 instructions and 411 to 341 registers.
+    // The group form takes it where it runs two waves per SIMD, whose registers cannot hold
+    // the i c^[i] history; at one wave its step is 2.6 % slower with it (6 bodies).
     bool literal_pow = true;
 
     // Events (unrolled form): the event op-list, whose rows 0..n-1 are this system's state
@@ -3165,15 +3165,16 @@ std::string generate_quad_prelude(const Sys &S, int order, bool high_acc, int sp
 // lane q of a slot evaluating its q-th node. Per order, the state rows come first, then
 // the slots level by level, one wavefront-scope fence per level. Every coefficient lives
 // in the instance's LDS block:
-//   T[k][r] = fl[k * R + r]: orders 0..p-1 of the state variables (rows 0..n-1), a zero
-//     row (n), the nodes whose history a recurrence reads, and the constants and
-//     parameters a recurrence reads at higher (zero) orders; order p of the state rows
-//     and the zero row. The state rows are the layout the group kernels' state update,
-//     grid output and event code read.
-//   cur[c] = fl[P * R + n + 1 + c]: the current order of every state variable (c = i),
-//     the zero entry (c = n), every node (c = node + 1) and every constant or
-//     parameter (zero above order 0), read by the linear nodes, the products with a
-//     constant or parameter and the right-hand sides;
+//   T[k][r] = fl[k * R + r]: orders 0..p-1 of the state variables with a row (not of a
+//     variable whose right-hand side is another state variable: x' = v makes
+//     v^[k] = (k + 1) x^[k+1], so only v's orders 0 and p are stored), of the nodes
+//     whose history a recurrence reads, and of the constants and parameters a recurrence
+//     reads at higher (zero) orders; order p of the state rows. R is odd (row reads in
+//     pairs of orders then stay conflict-free). The state rows are the layout
+//     the group kernels' state update, grid output and event code read.
+//   cur[c]: the current order of the state variables, nodes, constants and parameters
+//     that the linear nodes, the products with a constant or parameter and the
+//     right-hand sides read, numbered without gaps, with a zero and a sink entry.
 //   sv[q]: the value of every constant and parameter.
 // A lane's operand rows come from per-lane tables loaded once into registers. Each
 // recurrence at order k is split into the terms that read orders below k only, emitted
@@ -3295,9 +3296,39 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
     for (int i = 0; i < n; ++i)
         if (!is_node(S.rhs[i])) scal_index(S.rhs[i]);
     const int NS = (int)scal.size();
+    // State variables derived from a right-hand side of another: v with x' = v alone, where no
+    // recurrence reads v's history. v's orders are those of x, v^[k] = (k + 1) x^[k+1], so
+    // they have no rows (21 of the 42 variables of J2 + variational equations, a fifth of the
+    // block); the lane that owns x owns v too and passes v^[k] on to x^[k+1] in a register.
+    // dvar[x] = v; the others, na of them, have rows arow[].
+    std::vector<int> dvar(n, -1), arow(n + 1, -1);
+    int na = 0;
+    {
+        std::vector<char> conv(n, 0), isv(n, 0);
+        for (int j = n; j < NN; ++j)
+            if (kind[j] != WK_LIN && kind[j] != WK_MULS)
+                for (auto a : S.args[j])
+                    if (is_node(a) && (int)HYX_OPERAND_INDEX(a) < n) conv[HYX_OPERAND_INDEX(a)] = 1;
+        for (int x = 0; x < n; ++x) {
+            const int v = (int)HYX_OPERAND_INDEX(S.rhs[x]);
+            if (!is_node(S.rhs[x]) || v >= n || v == x || conv[v] || isv[v] || isv[x] || dvar[v] >= 0) continue;
+            dvar[x] = v;
+            isv[v] = 1;
+        }
+        for (int x = 0; x < n; ++x)
+            if (!isv[x]) arow[x] = na++;
+        arow[n] = na;
+    }
+    const bool derived = na < n;
+    const int own_a = (na + G - 1) / G, own = derived ? 2 * own_a : own_a;
+    if ((n + G - 1) / G > 8) {
+        why = "too many state variables per lane";
+        return "";
+    }
     // T rows and cur entries.
+    // (Slots without a variable use row na, a node's: it is written after them at every order.)
     std::vector<int> hrow(NN, -1);
-    int R = n + 1;
+    int R = na;
     for (int j = n; j < NN; ++j)
         if (hist[j]) hrow[j] = R++;
     // Constants and parameters: a T row only where a recurrence reads their higher
@@ -3307,36 +3338,13 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
         if (kind[j] != WK_LIN && kind[j] != WK_MULS)
             for (auto a : S.args[j])
                 if (!is_node(a) && srow[scal_index(a)] < 0) srow[scal_index(a)] = R++;
-    // A sink row: the T stores of slot lanes whose node has no history row go there, so
-    // a slot stores without a per-lane branch (nothing reads it).
-    const int sink = R++;
-    // T holds orders 0..P-1 of every row and order P of the state rows (and the zero row):
-    // node coefficients are formed up to order P-1.
-    const int CB = P * R + n + 1;
-    const int NC = NN + 1 + NS + 1; // the last entry is a sink, like the sink row
-    const int csink = NN + 1 + NS;
-    const int SVB = CB + NC;
-    const int flat = SVB + NS;
-    const int ipb = 64 / G;
-    if ((long)flat * ipb * 8 > 160 * 1024) {
-        why = "the coefficient rows exceed the 160 KB of LDS of a compute unit";
-        return "";
-    }
-    auto trow = [&](uint32_t w) -> int {
-        const int idx = (int)HYX_OPERAND_INDEX(w);
-        if (!is_node(w)) {
-            if (srow[scal_index(w)] < 0) throw std::logic_error("wave form: constant without a row");
-            return srow[scal_index(w)];
-        }
-        if (idx < n) return idx;
-        if (hrow[idx] < 0) throw std::logic_error("wave form: operand without a history row");
-        return hrow[idx];
-    };
-    auto cid = [&](uint32_t w) -> int {
-        const int idx = (int)HYX_OPERAND_INDEX(w);
-        if (!is_node(w)) return NN + 1 + scal_index(w);
-        return idx < n ? idx : idx + 1;
-    };
+    // A sink: the T stores of slot lanes whose node has no history row go there, so a slot
+    // stores without a per-lane branch: row 0 of the order after, a state variable's, which its owner
+    // stores before anybody reads it.
+    // Rows of consecutive orders are an odd number of doubles apart: one LDS instruction reads
+    // two orders of a row, and at a multiple of the banks the two would meet in one bank.
+    R = std::max(R, na + 1) | 1;
+    const int sink = R;
     // Levels. A node's level lies between its earliest, 1 + the highest earliest level of
     // its node operands, and its latest, 1 below the lowest latest level of the nodes that
     // read it (the last level for the nodes only right-hand sides read). Levels are
@@ -3486,12 +3494,193 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
                 }
             }
         }
-    const int own = (n + G - 1) / G;
-    if (own > 8) {
-        why = "too many state variables per lane";
+    // T holds orders 0..P-1 of every row and order P of the state rows (and the zero row):
+    // node coefficients are formed up to order P-1.
+    // Orders 0 and P of the derived state variables: VB + the row of the variable they follow.
+    const int VB = P * R + na + 1;
+    const int CB = VB + (derived ? 2 * (na + 1) : 0);
+    // The cur entries that somebody reads: operands of linear nodes and of products with
+    // constants (a derived node reads its source from a register), right-hand sides; and the
+    // zero entry, and a sink for the stores of lanes whose value nobody reads.
+    std::vector<char> cur_read(NN + 1 + NS, 0);
+    auto raw_cid = [&](uint32_t w) -> int {
+        const int idx = (int)HYX_OPERAND_INDEX(w);
+        if (!is_node(w)) return NN + 1 + scal_index(w);
+        return idx < n ? idx : idx + 1;
+    };
+    for (int j = n; j < NN; ++j) {
+        if (kind[j] == WK_LIN)
+            for (auto a : S.args[j]) {
+                if (!(dsrc[j] >= 0 && is_node(a))) cur_read[raw_cid(a)] = 1;
+            }
+        else if (kind[j] == WK_MULS && dsrc[j] < 0)
+            cur_read[raw_cid(is_node(S.args[j][0]) ? S.args[j][0] : S.args[j][1])] = 1;
+    }
+    for (int i = 0; i < n; ++i)
+        if (dvar[i] < 0) cur_read[raw_cid(S.rhs[i])] = 1;
+    cur_read[n] = 1;
+    // The pool (below) takes the products, squares and pows, whose sums over the orders below
+    // k are computed away from their slots. They are passed on through the place of the
+    // node's own order k: its T row, if all nodes of its slot have one (in_t), else its cur entry;
+    // pow nodes have a second sum, in an entry of its own.
+    const bool pooled = split_min == 0;
+    auto in_pool = [&](size_t s) {
+        return pooled && (slots[s].kind == WK_MUL || slots[s].kind == WK_SQ || slots[s].kind == WK_POW);
+    };
+    std::vector<char> in_t(slots.size(), 0);
+    for (size_t s = 0; s < slots.size(); ++s) {
+        if (!in_pool(s)) continue;
+        in_t[s] = 1;
+        for (auto j : slots[s].nodes) in_t[s] = in_t[s] && hist[j];
+        for (auto j : slots[s].nodes) cur_read[j + 1] = cur_read[j + 1] || !in_t[s];
+    }
+    auto trow = [&](uint32_t w) -> int {
+        const int idx = (int)HYX_OPERAND_INDEX(w);
+        if (!is_node(w)) {
+            if (srow[scal_index(w)] < 0) throw std::logic_error("wave form: constant without a row");
+            return srow[scal_index(w)];
+        }
+        if (idx < n) return arow[idx];
+        if (hrow[idx] < 0) throw std::logic_error("wave form: operand without a history row");
+        return hrow[idx];
+    };
+    // The pool's sums: rows a and b (for pow's second sum, w, the first is the weighted one).
+    struct PoolSum {
+        int node, a, b, w;
+        size_t slot;
+    };
+    std::vector<PoolSum> es;
+    for (size_t s = 0; s < slots.size(); ++s)
+        for (auto j : slots[s].nodes) {
+            if (!in_pool(s)) continue;
+            const int kd = slots[s].kind, a = trow(S.args[j][0]);
+            const int b = kd == WK_MUL ? trow(S.args[j][1]) : kd == WK_SQ ? a : hrow[j];
+            es.push_back({(int)j, a, b, 0, s});
+        }
+    for (size_t e = 0, n0 = es.size(); e < n0; ++e)
+        if (slots[es[e].slot].kind == WK_POW) es.push_back({es[e].node, es[e].b, es[e].a, 1, es[e].slot});
+    {
+        // Rows and pool lanes, placed to spread the LDS accesses over the banks: 16 lanes are
+        // served at once, a double at word x in the double bank x mod 16, so lanes with different
+        // rows that agree mod 16 serialise (at every order alike: they read the same one). A
+        // deterministic local search over swaps of rows (state variables' among themselves, the
+        // others' among themselves) and of sums between lanes. Measured (J2 + variational, 32
+        // lanes per instance, 32,768 instances to t = 17.5): SQ_LDS_BANK_CONFLICT 1.97e9 ->
+        // 1.47e9, kernel 16.9 -> 16.4 ms.
+        std::vector<std::pair<std::vector<int>, int>> acc; // (row per lane, accesses per step)
+        auto add = [&](auto fn, size_t cnt, int weight) {
+            std::vector<int> v;
+            for (size_t q = 0; q < cnt; ++q) v.push_back(fn(q));
+            acc.push_back({v, weight});
+        };
+        const int conv = (P - 1) * (P - 2) / 2;
+        const size_t npool = (es.size() + G - 1) / G;
+        for (size_t u = 0; u < npool; ++u) {
+            const size_t cnt = std::min<size_t>(G, es.size() - u * G);
+            add([&](size_t q) { return es[u * G + q].a; }, cnt, conv);
+            add([&](size_t q) { return es[u * G + q].b; }, cnt, conv);
+        }
+        for (size_t s = 0; s < slots.size(); ++s) {
+            const auto &nd = slots[s].nodes;
+            if (slots[s].kind == WK_LIN || slots[s].kind == WK_MULS || slots[s].kind == WK_TIME) continue;
+            add([&](size_t q) { return trow(S.args[nd[q]][0]); }, nd.size(), 2 * P);
+            if (slots[s].kind == WK_MUL || slots[s].kind == WK_DIV)
+                add([&](size_t q) { return trow(S.args[nd[q]][1]); }, nd.size(), 2 * P);
+            if (in_t[s]) add([&](size_t q) { return hrow[nd[q]]; }, nd.size(), 2 * P);
+        }
+        std::vector<int> pos(R); // place of each row
+        for (int r = 0; r < R; ++r) pos[r] = r;
+        auto cost1 = [&](size_t i) {
+            long tot = 0;
+            const auto &v = acc[i].first;
+            for (size_t q0 = 0; q0 < v.size(); q0 += 16) {
+                int worst = 0, cnt[16] = {0};
+                for (size_t q = q0; q < std::min(v.size(), q0 + 16); ++q) {
+                    bool dup = false;
+                    for (size_t z = q0; z < q; ++z) dup = dup || v[z] == v[q];
+                    if (!dup) worst = std::max(worst, ++cnt[pos[v[q]] & 15]);
+                }
+                tot += worst - 1;
+            }
+            return tot * acc[i].second;
+        };
+        std::vector<long> cost(acc.size());
+        for (size_t i = 0; i < acc.size(); ++i) cost[i] = cost1(i);
+        uint64_t rs = 0x9e3779b97f4a7c15ull;
+        auto rnd = [&](size_t k) {
+            rs = rs * 6364136223846793005ull + 1442695040888963407ull;
+            return (size_t)((rs >> 33) % (uint64_t)k);
+        };
+        auto try_move = [&](const std::vector<int> &touched, auto apply) {
+            long before = 0, after = 0;
+            std::vector<long> nc;
+            for (int i : touched) before += cost[i];
+            apply();
+            for (int i : touched) {
+                nc.push_back(cost1(i));
+                after += nc.back();
+            }
+            if (after > before)
+                apply(); // a swap undoes itself
+            else
+                for (size_t q = 0; q < touched.size(); ++q) cost[touched[q]] = nc[q];
+        };
+        for (int it = 0; it < 6000 && es.size() > 1; ++it) {
+            if (it & 1) {
+                const size_t x = rnd(es.size()), y = rnd(es.size()), ux = x / G, uy = y / G;
+                if (x == y || (ux != uy && (es[x].w || es[y].w))) continue;
+                std::vector<int> t{(int)(2 * ux), (int)(2 * ux + 1)};
+                if (uy != ux) t.insert(t.end(), {(int)(2 * uy), (int)(2 * uy + 1)});
+                try_move(t, [&]() {
+                    std::swap(es[x], es[y]);
+                    std::swap(acc[2 * ux].first[x % G], acc[2 * uy].first[y % G]);
+                    std::swap(acc[2 * ux + 1].first[x % G], acc[2 * uy + 1].first[y % G]);
+                });
+            } else {
+                const size_t x = rnd(R);
+                const size_t y = (int)x < na ? rnd(na) : na + rnd(R - na);
+                if (x == y) continue;
+                std::vector<int> t;
+                for (size_t i = 0; i < acc.size(); ++i)
+                    for (int r : acc[i].first)
+                        if (r == (int)x || r == (int)y) {
+                            t.push_back((int)i);
+                            break;
+                        }
+                try_move(t, [&]() { std::swap(pos[x], pos[y]); });
+            }
+        }
+        for (int i = 0; i < n; ++i)
+            if (arow[i] >= 0) arow[i] = pos[arow[i]];
+        for (auto *rows : {&hrow, &srow})
+            for (int &r : *rows)
+                if (r >= 0) r = pos[r];
+        for (auto &e : es) {
+            e.a = pos[e.a];
+            e.b = pos[e.b];
+        }
+    }
+    int NC = 0;
+    std::vector<int> centry(NN + 1 + NS, -1);
+    for (size_t c = 0; c < centry.size(); ++c)
+        if (cur_read[c]) centry[c] = NC++;
+    const int csink = NC++, czero = centry[n];
+    std::map<int, int> kqentry;
+    for (int j = n; j < NN && pooled; ++j)
+        if (kind[j] == WK_POW) kqentry[j] = NC++;
+    auto cstore = [&](int c) { return centry[c] >= 0 ? centry[c] : csink; };
+    const int SVB = CB + NC;
+    const int flat = SVB + NS;
+    const int ipb = 64 / G;
+    if ((long)flat * ipb * 8 > 160 * 1024) {
+        why = "the coefficient rows exceed the 160 KB of LDS of a compute unit";
         return "";
     }
-
+    auto cid = [&](uint32_t w) -> int {
+        const int c = centry[raw_cid(w)];
+        if (c < 0) throw std::logic_error("wave form: an operand without a current entry");
+        return c;
+    };
     // Per-lane tables: int fields w[f][g], double fields d[f][g].
     std::vector<std::vector<int>> W;
     std::vector<std::vector<double>> D;
@@ -3505,15 +3694,40 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
         D.push_back(v);
         return (int)D.size() - 1;
     };
-    std::vector<int> vo((size_t)G * own, -1);
-    for (int i = 0; i < n; ++i) vo[(size_t)(i % G) * own + i / G] = i;
-    // Right-hand side of each owned variable: its cur entry (the zero entry for none).
-    std::vector<int> f_rhs(own);
+    std::vector<int> vo((size_t)G * own, -1), vc((size_t)G * own, na);
+    for (int i = 0; i < n; ++i) {
+        if (arow[i] < 0) continue;
+        const size_t at = (size_t)(arow[i] % G) * own + arow[i] / G;
+        vo[at] = i;
+        vc[at] = arow[i];
+        if (dvar[i] >= 0) {
+            vo[at + own_a] = dvar[i];
+            vc[at + own_a] = arow[i];
+        }
+    }
+    // Right-hand side of each owned variable: its cur entry (the zero entry for none). Where a
+    // slot's variables have derived ones, its own orders come from theirs (f_rhs of slot own_a
+    // + o); in a mixed slot the lanes choose (f_der).
+    // f_cur: the entry a variable's own current order goes to (-1: none is read).
+    std::vector<int> f_rhs(own, -1), f_cur(own, -1), f_der(own, -1);
     for (int o = 0; o < own; ++o) {
-        std::vector<int> v(G, n);
-        for (int g = 0; g < G; ++g)
-            if (vo[(size_t)g * own + o] >= 0) v[g] = cid(S.rhs[vo[(size_t)g * own + o]]);
-        f_rhs[o] = addw(v);
+        std::vector<int> v(G, czero), c(G, csink), d(G, 0);
+        bool cany = false, any = false, all = true;
+        for (int g = 0; g < G; ++g) {
+            const int i = vo[(size_t)g * own + o];
+            if (i < 0) continue;
+            if (o >= own_a || dvar[i] < 0) {
+                v[g] = cid(S.rhs[i]);
+                any = true;
+            }
+            d[g] = o < own_a && dvar[i] >= 0;
+            all = all && d[g];
+            c[g] = cstore(i);
+            cany = cany || c[g] != csink;
+        }
+        if (any) f_rhs[o] = addw(v);
+        if (cany) f_cur[o] = addw(c);
+        if (o < own_a && derived && !all) f_der[o] = addw(d);
     }
 
     std::ostringstream h, o;
@@ -3522,6 +3736,10 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
       << "\n#define HYX_OWN " << own << "\n#define HYX_NX " << R << "\n#define HYX_XB 0\n#define HYX_FLAT " << flat
       << "\n#define HYX_WAVE_SLOTS " << slots.size() << "\n#define HYX_VO(o) hyx_wtab_vo[g * HYX_OWN + (o)]\n";
     if ((long)(flat + 14) * ipb * 8 > 160 * 1024) h << "#define HYX_REC_REGS 1\n";
+    // Two waves per SIMD where the LDS holds more than one block per SIMD: the levels are bound by
+    // LDS latency and throughput, so every block that the LDS can hold should run (J2 + variational, 23.0 KB
+    // per block: seven per CU).
+    if (!E && (long)(flat + 14) * ipb * 8 * 5 <= 160 * 1024) h << "#define HYX_GROUP_WAVES 2\n";
     h << "typedef unsigned long long hyx_u64;\n";
     h << "#ifndef HYX_CPU_EMU\n"
          "// A block is one wavefront, and the LDS operations of a wavefront complete in issue\n"
@@ -3531,6 +3749,10 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
          "    __builtin_amdgcn_fence(__ATOMIC_RELEASE, \"wavefront\");\n"
          "    __builtin_amdgcn_wave_barrier();\n"
          "    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");\n}\n"
+         "#define HYX_EMU_SYNC()\n"
+         "#define HYX_OPAQUE(x) __asm__ volatile(\"\" : \"+v\"(x))\n"
+         "#else\n"
+         "#define HYX_OPAQUE(x)\n"
          "#endif\n";
     h << group_fold_src();
 
@@ -3540,19 +3762,11 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
     };
     auto cur = [&](const std::string &c) { return "fl[" + std::to_string(CB) + " + " + c + "]"; };
     struct SlotTab {
-        int a = -1, b = -1, oc = -1, orow = -1, sgn = -1, al = -1, al1 = -1, cosf = -1;
+        int a = -1, b = -1, oc = -1, orow = -1, sgn = -1, al = -1, al1 = -1, cosf = -1, kq = -1;
         std::vector<int> lin;
         bool cur_any = false, hist_any = false;
     };
     std::vector<SlotTab> st(slots.size());
-    // Readers of each node's cur entry: linear nodes and right-hand sides (a derived node
-    // reads its source from a register).
-    std::vector<char> cur_read(NC, 0);
-    for (int j = n; j < NN; ++j)
-        if (kind[j] == WK_LIN || kind[j] == WK_MULS)
-            for (auto a : S.args[j])
-                if (!(dsrc[j] >= 0 && is_node(a))) cur_read[cid(a)] = 1;
-    for (int i = 0; i < n; ++i) cur_read[cid(S.rhs[i])] = 1;
     // Derived steps of each slot (the shape is the slot's; lanes past its width repeat the
     // first lane's, like its node): a product's constant per lane (d-field), a linear
     // node's constant operands per lane (their cur entries, read at order 0 only: they are
@@ -3577,13 +3791,13 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
             t.hist_any = t.hist_any || hist[j];
             t.cur_any = t.cur_any || cur_read[j + 1];
         }
-        if (t.cur_any) t.oc = addw(lanes([&](uint32_t j) { return (int)j + 1; }));
+        if (t.cur_any) t.oc = addw(lanes([&](uint32_t j) { return cstore((int)j + 1); }));
         if (t.hist_any) t.orow = addw(lanes([&](uint32_t j) { return hist[j] ? hrow[j] : sink; }));
         switch (sl.kind) {
         case WK_LIN: {
             for (int q = 0; q < sl.m; ++q)
                 t.lin.push_back(addw(lanes([&](uint32_t j) {
-                    return q < (int)S.args[j].size() ? cid(S.args[j][q]) : n;
+                    return q < (int)S.args[j].size() ? cid(S.args[j][q]) : czero;
                 })));
             t.sgn = addw(lanes([&](uint32_t j) {
                 int m = 0;
@@ -3651,11 +3865,55 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
                 ds.op = std::atoi(shp.c_str() + 1);
                 const std::string pat = shp.substr(shp.find(':') + 1);
                 for (size_t q = 0; q < pat.size(); ++q)
-                    ds.cterm.push_back(pat[q] == 'n' ? -1 : addw(dl([&](int x) { return x < 0 ? n : cid(S.args[x][q]); })));
+                    ds.cterm.push_back(pat[q] == 'n' ? -1 : addw(dl([&](int x) { return x < 0 ? czero : cid(S.args[x][q]); })));
             }
-            if (ds.cur_any) ds.oc = addw(dl([&](int x) { return x >= 0 && cur_read[x + 1] ? x + 1 : csink; }));
+            if (ds.cur_any) ds.oc = addw(dl([&](int x) { return x >= 0 ? cstore(x + 1) : csink; }));
             if (ds.hist_any) ds.orow = addw(dl([&](int x) { return x >= 0 && hist[x] ? hrow[x] : sink; }));
             dst[s].push_back(ds);
+        }
+    }
+    // The pool. A recurrence sum_{q=0..k} a^[q] b^[k-q] at order k has two terms with order-k
+    // factors, which wait for the node's level; the k - 1 others read lower orders only, and
+    // depend on no level. They are the bulk of the step's arithmetic and LDS reads, and evaluated in
+    // the nodes' slots, which the levels leave two thirds empty, they cost as much as full ones. So
+    // they are spread over all lanes, densely, whatever the nodes' levels: J2 + variational has
+    // 110 sums, 4 pool slots of 32 lanes instead of 9 slots (LDS reads and writes per step 4,090 ->
+    // 2,960 doubles per lane, kernel 19.3 -> 18.2 ms where the LDS was the bound, and the registers
+    // to run it without spills). Lane q of pool slot u sums the
+    // products of rows pa and pb (pw: the first one's orders weighted by their index, for
+    // pow's second sum). The terms with both factors below order k - 1 are spread over the levels
+    // of order k - 1, where they fill the waits of the exchanges; order k starts with the last two
+    // and stores the sums (po: T row or cur entry, by pt).
+    struct Pool {
+        int pa = -1, pb = -1, po = -1, pt = -1, pw = -1;
+    };
+    std::vector<Pool> pool;
+    if (pooled) {
+        for (size_t e0 = 0; e0 < es.size(); e0 += G) {
+            auto fld = [&](auto fn) {
+                std::vector<int> v(G, 0);
+                bool any = false;
+                for (int q = 0; q < G; ++q) {
+                    v[q] = fn(es[e0 + q < es.size() ? e0 + q : e0]);
+                    any = any || v[q] != 0;
+                }
+                return std::make_pair(addw(v), any);
+            };
+            Pool u;
+            u.pa = fld([](const PoolSum &e) { return e.a; }).first;
+            u.pb = fld([](const PoolSum &e) { return e.b; }).first;
+            u.po = fld([&](const PoolSum &e) { return e.w ? kqentry[e.node] : in_t[e.slot] ? hrow[e.node] : centry[e.node + 1]; }).first;
+            u.pt = fld([&](const PoolSum &e) { return e.w ? 0 : (int)in_t[e.slot]; }).first;
+            const auto w = fld([](const PoolSum &e) { return e.w; });
+            if (w.second) u.pw = w.first;
+            pool.push_back(u);
+        }
+        for (size_t s = 0; s < slots.size(); ++s) {
+            if (slots[s].kind != WK_POW) continue;
+            const int w = (int)slots[s].nodes.size();
+            std::vector<int> v(G, 0);
+            for (int q = 0; q < G; ++q) v[q] = kqentry[(int)slots[s].nodes[q < w ? q : 0]];
+            st[s].kq = addw(v);
         }
     }
     // Table fields are unsigned 8-bit values, four per 32-bit word, when every value fits
@@ -3669,7 +3927,7 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
         }
     const int tb_per = 32 / tb_bits;
     auto wv = [tb_bits, tb_per](int f) {
-        const std::string w = "tab.w[" + std::to_string(f / tb_per) + "]";
+        const std::string w = "w" + std::to_string(f / tb_per);
         const int sh = tb_bits * (f % tb_per);
         if (sh + tb_bits == 32) return "(int)((unsigned)" + w + " >> " + std::to_string(sh) + ")";
         return "(int)(((unsigned)" + w + " >> " + std::to_string(sh) + ") & " + std::to_string((1u << tb_bits) - 1) + "u)";
@@ -3707,9 +3965,46 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
     // overlap the previous level's exchange. Results in ko<s> (and kq<s>).
     // Returns whether ko<s> holds a value.
     std::vector<char> has_old(slots.size(), 0);
+    auto pl = [](size_t u, const char *nm, int k) { return std::string(nm) + std::to_string(u) + "_" + std::to_string(k); };
+    // The term of orders q and r in pool slot u's sum of order q + r.
+    auto pterm = [&](size_t u, int q, int r, bool first) {
+        const std::string acc = pl(u, "ps", q + r), b = Tk(wv(pool[u].pb), r);
+        std::string a = Tk(wv(pool[u].pa), q);
+        if (pool[u].pw >= 0 && q > 1) a = "((pw" + std::to_string(u) + " ? " + lit((double)q) + " : 1.0) * " + a + ")";
+        if (first)
+            o << "    double " << acc << " = " << a << " * " << b << ";\n";
+        else
+            o << "    " << acc << " = __builtin_fma(" << a << ", " << b << ", " << acc << ");\n";
+    };
+    // The start of order k: the newest orders join the sums, which then leave for LDS.
+    auto pool_close = [&](int k) {
+        for (size_t u = 0; u < pool.size() && k >= 2; ++u) {
+            pterm(u, k - 1, 1, k < 4);
+            if (k > 2) pterm(u, 1, k - 1, false);
+        }
+    };
+    auto pool_store = [&](int k) {
+        for (size_t u = 0; u < pool.size(); ++u)
+            o << "    fl[" << wv(pool[u].po) << " + (" << wv(pool[u].pt) << " ? " << k * R << " : " << CB << ")] = "
+              << pl(u, "ps", k) << ";\n";
+    };
+    // Level l of nl's part of the sums of order k + 1 over the orders 2 .. k - 1: one pool slot
+    // per level in turn, several terms at once (their LDS reads pair up).
+    auto pool_part = [&](int k, int l, int nl) {
+        const int np = (int)pool.size(), cnt = k - 2;
+        for (int u = 0; u < np; ++u) {
+            if (nl >= np && l % np != u) continue;
+            const int turns = nl >= np ? (nl - u + np - 1) / np : nl, t = nl >= np ? l / np : l;
+            for (int i = cnt * t / turns; i < cnt * (t + 1) / turns; ++i) pterm((size_t)u, 2 + i, k - 1 - i, i == 0);
+        }
+    };
     auto emit_old = [&](size_t s, int k) {
         const auto &sl = slots[s];
         const auto &t = st[s];
+        if (in_pool(s)) {
+            has_old[s] = k >= 2;
+            return;
+        }
         const std::string a = t.a >= 0 ? wv(t.a) : "", b = t.b >= 0 ? wv(t.b) : "";
         const std::string c = t.orow >= 0 ? wv(t.orow) : "";
         std::vector<std::pair<std::string, std::string>> tm, tm2;
@@ -3771,7 +4066,8 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
         const std::string a = t.a >= 0 ? wv(t.a) : "", b = t.b >= 0 ? wv(t.b) : "";
         const std::string c = t.orow >= 0 ? wv(t.orow) : "";
         const bool old = has_old[s] != 0;
-        const std::string O = ko(s);
+        const bool pool_sum = old && in_pool(s);
+        const std::string O = !pool_sum ? ko(s) : in_t[s] ? Tk(c, k) : cur(wv(t.oc));
         o << "    {\n";
         switch (sl.kind) {
         case WK_LIN: {
@@ -3797,10 +4093,13 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
             if (k == 0)
                 o << "        const double v = " << Tk(a, 0) << " * " << Tk(a, 0) << ";\n";
             else {
+                // (The pool sums both halves of a square.)
                 o << "        const double acc = "
-                  << (old ? "__builtin_fma(" + Tk(a, 0) + ", " + Tk(a, k) + ", " + O + ")" : Tk(a, 0) + " * " + Tk(a, k))
+                  << (old && !pool_sum ? "__builtin_fma(" + Tk(a, 0) + ", " + Tk(a, k) + ", " + O + ")" : Tk(a, 0) + " * " + Tk(a, k))
                   << ";\n";
-                if (k % 2)
+                if (pool_sum)
+                    o << "        const double v = __builtin_fma(2.0, acc, " << O << ");\n";
+                else if (k % 2)
                     o << "        const double v = acc + acc;\n";
                 else
                     o << "        const double v = __builtin_fma(" << Tk(a, k / 2) << ", " << Tk(a, k / 2) << ", acc + acc);\n";
@@ -3818,7 +4117,8 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
                 if (k == 1)
                     o << "        const double v = s1 * " << rv(s, "raa") << ";\n";
                 else
-                    o << "        const double v = __builtin_fma(s1, " << rv(s, "raa") << ", -(" << kq(s) << " * " << rv(s, "rab")
+                    o << "        const double v = __builtin_fma(s1, " << rv(s, "raa") << ", -("
+                      << (pool_sum ? cur(wv(t.kq)) : kq(s)) << " * " << rv(s, "rab")
                       << ") * " << lit(1.0 / k) << ");\n";
             }
             break;
@@ -3867,6 +4167,8 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
             break;
         case WK_TIME: o << "        const double v = " << (k == 0 ? "t0" : k == 1 ? "1.0" : "0.0") << ";\n"; break;
         }
+        // (Lanes past the slot's width read the same sum: on the CPU, before the first writes.)
+        if (pool_sum) o << "        HYX_EMU_SYNC();\n";
         if (t.cur_any) o << "        " << cur(wv(t.oc)) << " = v;\n";
         if (t.hist_any) o << "        " << Tk(wv(t.orow), k) << " = v;\n";
         // Derived steps: the recurrences of the nodes they replace (a product with a
@@ -3906,6 +4208,7 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
             if (k > 0)
                 for (size_t s = 0; s < slots.size(); ++s)
                     if (slvl[s] == l + 1) emit_old(s, k);
+            if (k + 1 < P && pooled) pool_part(k, l - 1, maxlv);
             for (size_t s = s0; s < slots.size() && slvl[s] == l; ++s) emit_new(s, k);
             while (s0 < slots.size() && slvl[s0] == l) ++s0;
             o << "    hyx_wsync();\n";
@@ -3937,18 +4240,24 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
         h << "__constant__ double hyx_wtab_d[" << df.size() << "] = {";
         for (size_t q = 0; q < df.size(); ++q) h << (q ? "," : "") << lit(df[q]);
         h << "};\n";
-        h << "__constant__ int hyx_wtab_vo[" << vo.size() << "] = {";
-        for (size_t q = 0; q < vo.size(); ++q) h << (q ? "," : "") << vo[q];
-        h << "};\n";
+        for (const auto &t : {std::make_pair("vo", &vo), std::make_pair("vc", &vc)}) {
+            h << "__constant__ int hyx_wtab_" << t.first << "[" << t.second->size() << "] = {";
+            for (size_t q = 0; q < t.second->size(); ++q) h << (q ? "," : "") << (*t.second)[q];
+            h << "};\n";
+        }
     }
     h << "__device__ __forceinline__ void hyx_gtab_load(hyx_gtab &t, int g)\n{\n"
-         "    for (int q = 0; q < HYX_OWN; ++q) { t.vo[q] = hyx_wtab_vo[g * HYX_OWN + q]; t.vc[q] = t.vo[q] >= 0 ? t.vo[q] : HYX_N; }\n";
+         "    for (int q = 0; q < HYX_OWN; ++q) { t.vo[q] = hyx_wtab_vo[g * HYX_OWN + q]; t.vc[q] = hyx_wtab_vc[g * HYX_OWN + q]; }\n";
     if (NWP) h << "    for (int f = 0; f < " << NWP << "; ++f) t.w[f] = hyx_wtab_w[f * HYX_G + g];\n";
     if (!D.empty()) h << "    for (int f = 0; f < " << D.size() << "; ++f) t.d[f] = hyx_wtab_d[f * HYX_G + g];\n";
     h << "}\n";
 
     h << "__device__ __forceinline__ double hyx_grow(const double *fl, const hyx_gtab &t, int o, int k)\n{\n"
-         "    return fl[HYX_XB + k * HYX_NX + t.vc[o]];\n}\n";
+      << (derived ? "    if (o >= " + std::to_string(own_a) + ") {\n        if (k == 0 || k == HYX_P) return fl[" +
+                        std::to_string(VB) + " + (k ? " + std::to_string(na + 1) +
+                        " : 0) + t.vc[o]];\n        return (double)(k + 1) * fl[HYX_XB + (k + 1) * HYX_NX + t.vc[o]];\n    }\n"
+                  : std::string())
+      << "    return fl[HYX_XB + k * HYX_NX + t.vc[o]];\n}\n";
 
     auto xv = [](int oo, int k) { return "x" + std::to_string(oo) + "_" + std::to_string(k); };
     auto vcol = [](int oo) { return "vc" + std::to_string(oo); };
@@ -3965,14 +4274,26 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
         if (kd == WK_SQRT) o << "    double " << rv(s, "rs") << " = 0.0;\n";
         if (kd == WK_LOG) o << "    double " << rv(s, "rl") << " = 0.0;\n";
     }
-    for (int oo = 0; oo < own; ++oo)
-        o << "    const int " << vcol(oo) << " = (tab.vo[" << oo << "] >= 0) ? tab.vo[" << oo << "] : HYX_N;\n";
+    for (int oo = 0; oo < own; ++oo) o << "    const int " << vcol(oo) << " = tab.vc[" << oo << "];\n";
+    // The table words, made opaque once per step: unpacked before the loop over steps, their
+    // fields hold 60 more registers in the persistent kernel and it spills (J2 + variational at two
+    // waves per SIMD: 16.4 ms with the spills, 13.75 ms unpacking once per step, without
+    // any; unpacking at every order, 21.5 ms).
+    for (size_t q = 0; q < NWP; ++q) o << "    int w" << q << " = tab.w[" << q << "];\n    HYX_OPAQUE(w" << q << ");\n";
+    for (size_t u = 0; u < pool.size(); ++u)
+        if (pool[u].pw >= 0) o << "    const bool pw" << u << " = " << wv(pool[u].pw) << " != 0;\n";
+    // Order k of slot oo: its T row, or (derived slots) the row it is read from, times (k + 1).
+    auto xrow = [&](int oo, int k) {
+        if (oo < own_a) return "fl[" + vcol(oo) + " + " + std::to_string(k * R) + "]";
+        if (k == 0 || k == P) return "fl[" + vcol(oo) + " + " + std::to_string(VB + (k ? na + 1 : 0)) + "]";
+        return "(" + lit((double)(k + 1)) + " * fl[" + vcol(oo) + " + " + std::to_string((k + 1) * R) + "])";
+    };
     o << "    hyx_wsync();\n";
     // Order 0: state rows, constants and parameters (lane 0), then the slots.
     for (int oo = 0; oo < own; ++oo) {
         o << "    const double " << xv(oo, 0) << " = xo[" << oo << "];\n";
-        o << "    fl[" << vcol(oo) << "] = " << xv(oo, 0) << ";\n";
-        o << "    " << cur(vcol(oo)) << " = " << xv(oo, 0) << ";\n";
+        o << "    " << xrow(oo, 0) << " = " << xv(oo, 0) << ";\n";
+        if (f_cur[oo] >= 0) o << "    " << cur(wv(f_cur[oo])) << " = " << xv(oo, 0) << ";\n";
     }
     if (NS) {
         o << "    if (g == 0) {\n";
@@ -3981,7 +4302,7 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
             const std::string val = HYX_OPERAND_KIND(w) == HYX_KIND_CONST ? lit(S.consts[HYX_OPERAND_INDEX(w)])
                                                                            : "pv[" + std::to_string(HYX_OPERAND_INDEX(w)) + "]";
             if (srow[q] >= 0) o << "        fl[" << srow[q] << "] = " << val << ";\n";
-            o << "        fl[" << (CB + NN + 1 + q) << "] = " << val << ";\n";
+            if (centry[NN + 1 + q] >= 0) o << "        fl[" << (CB + centry[NN + 1 + q]) << "] = " << val << ";\n";
             o << "        fl[" << (SVB + q) << "] = " << val << ";\n";
         }
         o << "    }\n";
@@ -3994,16 +4315,32 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
         if (k < P)
             for (size_t s = 0; s < slots.size(); ++s)
                 if (slvl[s] == 1) emit_old(s, k);
-        for (int oo = 0; oo < own; ++oo) o << "    const double r" << oo << "_" << k << " = " << cur(wv(f_rhs[oo])) << ";\n";
+        for (int oo = 0; oo < own; ++oo)
+            if (f_rhs[oo] >= 0) o << "    const double r" << oo << "_" << k << " = " << cur(wv(f_rhs[oo])) << ";\n";
+        if (pooled && k < P) pool_close(k);
         o << "    hyx_wsync();\n";
-        for (int oo = 0; oo < own; ++oo) {
-            o << "    const double " << xv(oo, k) << " = r" << oo << "_" << k << " * " << lit(1.0 / k) << ";\n";
-            o << "    fl[" << vcol(oo) << " + " << k * R << "] = " << xv(oo, k) << ";\n";
-            if (k < P) o << "    " << cur(vcol(oo)) << " = " << xv(oo, k) << ";\n";
+        for (int oo = own - 1; oo >= 0; --oo) {
+            // A variable with a derived one takes that one's order k - 1.
+            const std::string r = "r" + std::to_string(oo) + "_" + std::to_string(k);
+            std::string src = r;
+            if (derived && oo < own_a) {
+                const std::string d = xv(oo + own_a, k - 1);
+                src = f_der[oo] < 0 ? d : f_rhs[oo] < 0 ? d : "(" + wv(f_der[oo]) + " ? " + d + " : " + r + ")";
+            } else if (f_rhs[oo] < 0)
+                src = "0.0";
+            o << "    const double " << xv(oo, k) << " = " << src << " * " << lit(1.0 / k) << ";\n";
+            if (oo < own_a || k == P) o << "    " << xrow(oo, k) << " = " << xv(oo, k) << ";\n";
+            if (k < P && f_cur[oo] >= 0) o << "    " << cur(wv(f_cur[oo])) << " = " << xv(oo, k) << ";\n";
+        }
+        // (Lanes without a variable have just written to row na, on the GPU before these stores.)
+        if (pooled && k >= 2 && k < P) {
+            o << "    HYX_EMU_SYNC();\n";
+            pool_store(k);
         }
         if (k == 1 && NS) {
             o << "    if (g == 0) {\n";
-            for (int q = 0; q < NS; ++q) o << "        fl[" << (CB + NN + 1 + q) << "] = 0.0;\n";
+            for (int q = 0; q < NS; ++q)
+                if (centry[NN + 1 + q] >= 0) o << "        fl[" << (CB + centry[NN + 1 + q]) << "] = 0.0;\n";
             o << "    }\n";
         }
         o << "    hyx_wsync();\n";
@@ -4013,12 +4350,17 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
     for (int oo = 0; oo < own; ++oo) {
         o << "        if (tab.vo[" << oo << "] >= 0)\n";
         o << "            for (int k = 0; k <= HYX_P; ++k) tc[((hyx_u64)tab.vo[" << oo << "] * " << (P + 1)
-          << " + k) * tcs] = fl[HYX_XB + k * HYX_NX + " << vcol(oo) << "];\n";
+          << " + k) * tcs] = hyx_grow(fl, tab, " << oo << ", k);\n";
     }
     o << "    }\n";
     if (E) {
         Gen eg(*E, P, high_acc);
-        eg.lds_row = [&](uint32_t i, int k) { return "fl[" + std::to_string(k * R + (int)i) + "]"; };
+        eg.lds_row = [&](uint32_t i, int k) {
+            if (arow[i] >= 0) return "fl[" + std::to_string(k * R + arow[i]) + "]";
+            const int x = arow[(size_t)(std::find(dvar.begin(), dvar.end(), (int)i) - dvar.begin())];
+            if (k == 0 || k == P) return "fl[" + std::to_string(VB + (k ? na + 1 : 0) + x) + "]";
+            return "(" + lit((double)(k + 1)) + " * fl[" + std::to_string((k + 1) * R + x) + "])";
+        };
         o << "    double hyx_evg[" << nev << "][" << (P + 1) << "];\n    {\n";
         for (uint32_t j = E->n; j < E->nnodes; ++j) eg.order0(j);
         for (int k = 1; k <= P; ++k)
@@ -4062,23 +4404,35 @@ std::string generate_wave_prelude(const Sys &S, int P, bool high_acc, int G, con
         for (int oo = 0; oo < own; ++oo) {
             o << "            if (tab.vo[" << oo << "] >= 0)\n";
             o << "                for (int k = 0; k <= HYX_P; ++k) tc[((hyx_u64)tab.vo[" << oo << "] * " << (P + 1)
-              << " + k) * tcs] = fl[HYX_XB + k * HYX_NX + " << vcol(oo) << "];\n";
+              << " + k) * tcs] = hyx_grow(fl, tab, " << oo << ", k);\n";
         }
         o << "        }\n    }\n";
         o << "    hyx_mx = mx;\n";
     }
     o << "    int nf = 0;\n";
     for (int oo = 0; oo < own; ++oo) {
-        if (!high_acc) {
+        if (!high_acc && derived && oo < own_a) {
+            // The slot and its derived one in one pass over the rows.
+            const int d = oo + own_a;
+            o << "    { double r = " << xv(oo, P) << ", s = " << xv(d, P) << ", c = " << xv(oo, P) << ";\n";
+            for (int k = P - 1; k >= 0; --k)
+                o << "      s = __builtin_fma(s, h, " << (k == 0 ? xrow(d, 0) : lit((double)(k + 1)) + " * c") << "); c = "
+                  << xrow(oo, k) << "; r = __builtin_fma(r, h, c);\n";
+            for (int q : {oo, d})
+                o << "      xo[" << q << "] = tab.vo[" << q << "] >= 0 ? " << (q == oo ? "r" : "s") << " : 0.0; nf |= isfinite(xo[" << q
+                  << "]) ? 0 : 1;\n";
+            o << "    }\n";
+        } else if (!high_acc && !derived) {
             o << "    { double r = " << xv(oo, P) << ";\n";
-            o << "#pragma unroll\n      for (int k = HYX_P - 1; k >= 0; --k) r = __builtin_fma(r, h, fl[HYX_XB + k * HYX_NX + "
-              << vcol(oo) << "]);\n";
-        } else {
+            for (int k = P - 1; k >= 0; --k) o << "      r = __builtin_fma(r, h, " << xrow(oo, k) << ");\n";
+            o << "      xo[" << oo << "] = tab.vo[" << oo << "] >= 0 ? r : 0.0; nf |= isfinite(xo[" << oo << "]) ? 0 : 1; }\n";
+        } else if (high_acc) {
             o << "    { double r = " << xv(oo, 0) << ", cp = 0.0, hk = 1.0;\n";
-            o << "#pragma unroll\n      for (int k = 1; k <= HYX_P; ++k) { hk *= h; const double y = fl[HYX_XB + k * HYX_NX + "
-              << vcol(oo) << "] * hk - cp; const double tt = r + y; cp = (tt - r) - y; r = tt; }\n";
+            for (int k = 1; k <= P; ++k)
+                o << "      { hk *= h; const double y = " << xrow(oo, k)
+                  << " * hk - cp; const double tt = r + y; cp = (tt - r) - y; r = tt; }\n";
+            o << "      xo[" << oo << "] = tab.vo[" << oo << "] >= 0 ? r : 0.0; nf |= isfinite(xo[" << oo << "]) ? 0 : 1; }\n";
         }
-        o << "      xo[" << oo << "] = r; nf |= (tab.vo[" << oo << "] >= 0 && !isfinite(r)) ? 1 : 0; }\n";
     }
     o << "    nf_out = hyx_gany(nf) != 0;\n    h_out = h;\n}\n";
     return h.str() + o.str();

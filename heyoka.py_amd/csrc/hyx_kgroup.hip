@@ -12,9 +12,10 @@
 // coefficient histories in registers, and owns the state variables
 // tab.vo[o] (o < HYX_OWN). Per order, coefficients are exchanged through this
 // instance's LDS block `fl` of HYX_FLAT doubles: the cluster outputs of the
-// current order, a zero slot, and every order of every state variable
-// (rows of HYX_NX = n + 1 columns, one of them zero; variable tab.vo[o] sits in
-// column tab.vc[o]), which the state update reads.
+// current order, a zero slot, and the orders of the state variables, which the state
+// update reads (variable tab.vo[o] in column tab.vc[o]; order 0 in a row of HYX_NX
+// columns, the later ones HYX_RS apart; a variable that is another's derivative is read
+// from that one's next order).
 //
 // Every lane of the wave executes every step, also lanes whose group has no
 // instance (their results are not stored): hyx_gstep exchanges data between the

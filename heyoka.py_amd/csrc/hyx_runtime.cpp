@@ -135,14 +135,30 @@ std::string cache_dir()
     return lib_dir() + "/code_cache";
 }
 
-std::vector<std::string> rtc_options(const std::string &arch)
+std::vector<std::string> rtc_options(const std::string &arch, const std::string &src)
 {
-    return {"--offload-arch=" + arch, "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
+    std::vector<std::string> o = {"--offload-arch=" + arch, "-O3", "-std=c++17",
+                                  "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
+    // The wave form, without loop-invariant motion of machine instructions: in the persistent kernel's
+    // loop over steps it hoists literals and addresses of the whole step into registers, and at the
+    // 256 of two waves per SIMD 29 others spill (J2 + variational: 243 registers and no spill
+    // without it). The other forms keep it: hoisted literals shorten their steps (four
+    // pendulums 0.80 against 0.84 ms).
+    // And scheduled stage by stage within the occupancy that the kernel declares: ROCm 7.2's default
+    // scheduler gives up on these loops and leaves the reads of the LDS where the source has
+    // them, each right before its use and waited for by itself (805 waits for an empty queue in
+    // a step of J2 + variational against 211; 32,768 of them 16.6 against 13.75 ms, and a wave
+    // with its SIMD to itself 34 against 21.9 us a step). ROCm 7.0's default schedules them
+    // as this does.
+    if (src.find("#define HYX_WAVE 1\n") != std::string::npos)
+        o.insert(o.end(), {"-mllvm", "-disable-machine-licm", "-mllvm",
+                           "-misched=gcn-iterative-max-occupancy-experimental"});
+    return o;
 }
 
 int get_code(const std::string &src, const std::string &arch, std::vector<char> &code)
 {
-    const auto opts = rtc_options(arch);
+    const auto opts = rtc_options(arch, src);
     std::string keysrc = src;
     for (auto &o : opts) keysrc += "\n" + o;
     char kbuf[32];
