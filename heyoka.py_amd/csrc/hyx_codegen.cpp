@@ -2072,6 +2072,16 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
         return "fl[" + std::to_string(k == 0 ? xb : xb + nx + (k - 1) * rs) + " + " + col + "]";
     };
     auto vcol = [&](int oo) { return "vc" + std::to_string(oo); };
+    // Slots where some lane owns a variable without a derived one: that lane's derived slot is
+    // empty, but what it would derive is the integral of its variable, not zero. There the derived
+    // values are masked (slots whose lanes all have one, as N bodies alone, need no select).
+    std::vector<char> lone_owner((size_t)std::max(own_a, 1), 0);
+    for (int oo = 0; derived && oo < own_a; ++oo)
+        for (int g = 0; g < G; ++g)
+            if (gp.vo[(size_t)g * own + oo] >= 0 && gp.vo[(size_t)g * own + own_a + oo] < 0) lone_owner[(size_t)oo] = 1;
+    auto owned = [](int oo, const std::string &v) {
+        return "(tab.vo[" + std::to_string(oo) + "] >= 0 ? " + v + " : 0.0)";
+    };
     o << "template <bool WTC, class TAB>\n"
          "__device__ __forceinline__ void hyx_gstep(double (&xo)[HYX_OWN], const double (&pv)[HYX_NPAR], double t0, "
          "const double &max_dt, double &h_out, bool &nf_out, int g, double *fl, const TAB &tab, double *__restrict__ tc, "
@@ -2234,8 +2244,10 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
         // is not held in registers through the step).
         const bool d = oo >= own_a;
         const std::string x0 = derived ? X(0, vcol(oo)) : xv(oo, 0);
-        const std::string xp = d ? xv(oo - own_a, P - 1) + " * " + lit(1.0 / P) : xv(oo, P);
-        const std::string xq = d ? xv(oo - own_a, P - 2) + " * " + lit(1.0 / (P - 1)) : xv(oo, P - 1);
+        std::string xp = d ? xv(oo - own_a, P - 1) + " * " + lit(1.0 / P) : xv(oo, P);
+        std::string xq = d ? xv(oo - own_a, P - 2) + " * " + lit(1.0 / (P - 1)) : xv(oo, P - 1);
+        if (d && lone_owner[(size_t)(oo - own_a)])
+            for (std::string *v : {&xp, &xq}) *v = owned(oo, *v);
         o << "    mx = fmax(mx, fabs(" << x0 << "));\n";
         o << "    mo = fmax(mo, fabs(" << xp << "));\n";
         o << "    mom1 = fmax(mom1, fabs(" << xq << "));\n";
@@ -2287,6 +2299,7 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
                 o << "      c = " << X(k - 1, vcol(oo)) << "; r = __builtin_fma(r, h, c); s = __builtin_fma(s, h, c * "
                   << lit(1.0 / k) << ");\n";
             o << "      s = __builtin_fma(s, h, " << X(0, vcol(d)) << ");\n";
+            if (lone_owner[(size_t)oo]) o << "      s = " << owned(d, "s") << ";\n";
             o << "      xo[" << oo << "] = r; xo[" << d << "] = s; nf |= (isfinite(r) && isfinite(s)) ? 0 : 1; }\n";
         } else if (!high_acc) {
             o << "    { double r = " << xv(oo, P) << ";\n";
@@ -2300,6 +2313,7 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
             o << "      { hk *= h; const double y = "
               << (oo < own_a ? X(k, vcol(oo)) : "(" + X(k - 1, vcol(oo - own_a)) + " * " + lit(1.0 / k) + ")")
               << " * hk - cp; const double tt = r + y; cp = (tt - r) - y; r = tt; }\n";
+        if (oo >= own_a && lone_owner[(size_t)(oo - own_a)]) o << "      r = " << owned(oo, "r") << ";\n";
         o << "      xo[" << oo << "] = r; nf |= (tab.vo[" << oo << "] >= 0 && !isfinite(r)) ? 1 : 0; }\n";
     }
     o << "    nf_out = hyx_gany(nf) != 0;\n    h_out = h;\n}\n";
