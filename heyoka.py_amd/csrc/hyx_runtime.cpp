@@ -149,10 +149,11 @@ std::vector<std::string> rtc_options(const std::string &arch, const std::string 
     // them, each right before its use and waited for by itself (805 waits for an empty queue in
     // a step of J2 + variational against 211; 32,768 of them 16.6 against 13.75 ms, and a wave
     // with its SIMD to itself 34 against 21.9 us a step). ROCm 7.0's default schedules them
-    // as this does.
+    // as this does. By the option that takes any name: a compiler that does not know this scheduler
+    // uses its default, where an unknown value of -misched ends the process (LLVM's option
+    // parser exits). Every compiler with gfx950 has both options.
     if (src.find("#define HYX_WAVE 1\n") != std::string::npos)
-        o.insert(o.end(), {"-mllvm", "-disable-machine-licm", "-mllvm",
-                           "-misched=gcn-iterative-max-occupancy-experimental"});
+        o.insert(o.end(), {"-mllvm", "-disable-machine-licm", "-mllvm", "-amdgpu-sched-strategy=iterative-maxocc"});
     return o;
 }
 
