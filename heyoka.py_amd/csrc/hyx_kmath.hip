@@ -29,7 +29,8 @@ __device__ __forceinline__ double hyx_ipow(double y)
 // one, at most 4e-5, over R), and the error of an iteration is (R + 1) / 2 times the square of
 // the last, so two reach double precision; the rounding of q y^R enters y divided by R. q is scaled by
 // 2^(-R e) and y by 2^e, so that no power of y leaves the exponent range, whatever q.
-// den = 0 gives inf and den = inf gives 0, as pow() does.
+// den = 0 gives inf and den = inf gives 0, as pow() does; num / den beyond the largest double
+// (q below 2^-1024) gives inf too, as the division in pow(num / den, 1 / R) does.
 template <int R>
 __device__ __forceinline__ double hyx_root(double rnum, double den)
 {
@@ -55,8 +56,9 @@ __device__ __forceinline__ double hyx_root(double rnum, double den)
     double y = (double)y0;
     y = __builtin_fma(y * (1.0 / R), __builtin_fma(-qs, hyx_ipow<R>(y), 1.0), y);
     y = __builtin_fma(y * (1.0 / R), __builtin_fma(-qs, hyx_ipow<R>(y), 1.0), y);
-    // q = 0 or inf: the start is the value.
-    return (q == 0.0 || q == __builtin_inf()) ? (double)y0 : ldexp(y, -ei);
+    if (q <= 0x1p-1024) return __builtin_inf();
+    // q = inf: the start is the value.
+    return q == __builtin_inf() ? (double)y0 : ldexp(y, -ei);
 }
 
 // s ~ x^(-1/2) to about one ulp, and its correction: p + pl = s^2 exactly, and

@@ -57,6 +57,20 @@ def test_root_against_extended_precision(lib, r):
     assert f(1.0, 0.0) == np.inf and f(1.0, np.inf) == 0.0 and np.isnan(f(1.0, np.nan)) and f(0.0, 3.0) == np.inf
 
 
+@pytest.mark.parametrize("r", ROOTS)
+def test_root_of_an_overflowing_quotient(lib, r):
+    # num / den above the largest double: inf, as pow(num / den, 1 / r); just below it: finite.
+    f = getattr(lib, f"root_{r}")
+    f.restype, f.argtypes = ct.c_double, [ct.c_double] * 2
+    for num, den in [(1.0, 1e-310), (1.0, 5e-324), (1e10, 1e-300), (1e200, 1e-200), (1.0, 2.0 ** -1024)]:
+        with np.errstate(over="ignore"):
+            assert np.float64(num) / den == np.inf
+        assert f(1.0 / num, den) == np.inf, (num, den)
+    for num, den in [(1.0, 2.0 ** -1023), (1.0, 2.0 ** -1022), (2.0 ** 500, 2.0 ** -522)]:
+        ref = (np.longdouble(num) / den) ** (np.longdouble(1) / r)
+        assert abs(f(1.0 / num, den) / ref - 1) <= 2.0 ** -52 * (1 + 1 / r), (num, den)
+
+
 @pytest.mark.parametrize("name,al", [("m32", -1.5), ("m12", -0.5)])
 def test_half_integer_powers(lib, name, al):
     f = getattr(lib, name)
@@ -102,3 +116,24 @@ def test_step_size_over_the_exponent_range(amp):
     r = O.step_batch(hy.taylor_decompose(sys_), 19, st, max_dt=np.array([1e3]))
     assert int(ta.step_res[0][0]) == int(r["outcome"][0])
     assert abs(ta.last_h[0] - r["h"][0]) <= 1e-14 * abs(r["h"][0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["unrolled", "compact", "group", "wave"])
+@pytest.mark.parametrize("amp", [1e-300, 1e-290, 1e-280])
+def test_free_step_of_a_tiny_state(amp, form):
+    # Without a step limit: order 19 of a state of 1e-300 is 1e-317, whose quotient overflows (the step
+    # is infinite and its state not finite, as in the oracle); from 1e-290 on it does not.
+    x, y, vx, vy = hy.make_vars("x", "y", "vx", "vy")
+    sys_ = [(x, vx), (y, vy), (vx, -x * 1.5), (vy, -y * 1.5)]
+    if form == "group":
+        sys_ = [(x, vx), (y, vy), (vx, hy.sin(x) * -1.5), (vy, hy.sin(y) * -1.5)]
+    st = np.array([[amp], [0.5 * amp], [amp], [0.5 * amp]])
+    ta = hy.taylor_adaptive_batch(sys_, st, tol=1e-15, code_form=form)
+    ta.step()
+    r = O.step_batch(hy.taylor_decompose(sys_), 19, st)
+    assert int(ta.step_res[0][0]) == int(r["outcome"][0])
+    if np.isfinite(r["h"][0]):
+        assert abs(ta.last_h[0] - r["h"][0]) <= 1e-13 * abs(r["h"][0])
+    else:
+        assert ta.last_h[0] == r["h"][0]
