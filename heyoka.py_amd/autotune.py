@@ -77,6 +77,9 @@ def measure(system, state, pars, t_final, waves_per_cu, refill_min, repeats=1):
     N = state.shape[1]
     b = _lib.Batch(system, N)
     b.set_persistent_config(waves_per_cu, refill_min)
+    # The launch shape is the lane form's: no tail form, in which a sample of up to 128 instances
+    # per CU would run from its start, whatever the shape.
+    b.set_twin_tail(0)
     best = 0.0
     final = None
     for _ in range(repeats):

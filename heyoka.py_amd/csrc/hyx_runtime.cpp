@@ -1706,6 +1706,14 @@ int hyx_autotune(hyx_batch *b, const double *tf_hi, const char *cache_path, hyx_
         HIPCHK(hipStreamSynchronize(b->stream));
         return 0;
     };
+    // Without the tail form, in which a small batch would run from its start: the candidates are
+    // launch shapes of the lane form.
+    struct NoTail {
+        hyx_batch *b;
+        uint32_t tail_min;
+        explicit NoTail(hyx_batch *batch) : b(batch), tail_min(batch->tail_min) { b->tail_min = 0; }
+        ~NoTail() { b->tail_min = tail_min; }
+    } no_tail(b);
     const uint32_t waves[] = {0, 1, 2, 4, 8};
     const uint32_t refills[] = {1, 8, 32};
     hyx_tune_res top{0, 1, -1.0, 0};

@@ -266,7 +266,8 @@ int hyx_batch_last_timing(const hyx_batch *b, double *kernel_ms, uint64_t *launc
  * end; 0 when no instance was handed off. */
 int hyx_batch_last_tail_ms(const hyx_batch *b, double *tail_ms);
 /* Persistent-form tuning: waves per CU (0 = occupancy limit) and the idle-lane
- * count that triggers a refill (1..64). */
+ * count that triggers a refill (1..64). A batch that starts in its tail form (see
+ * hyx_batch_set_twin_tail) launches one wave per 64 lanes it needs instead; the refill count holds. */
 int hyx_batch_set_persistent_config(hyx_batch *b, uint32_t waves_per_cu, uint32_t refill_min);
 /* Persistent form: iterations one instance may take per launch before it is
  * written back and the kernel relaunched (default 65536). Bounds the duration of

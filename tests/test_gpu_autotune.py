@@ -89,3 +89,31 @@ def test_autotune_instances_per_wavefront(tmp_path, monkeypatch):
     finals = [AT.measure(get_system(dec, 19, compact=f), wl.state, None, tf, 0, 1)[1] for f in forms]
     for f in finals[1:]:
         assert np.array_equal(f, finals[0])
+
+
+@pytest.mark.parametrize("n", [300, 4000])
+def test_tuners_time_the_lane_form(n, tmp_path, monkeypatch):
+    # The launch shape is the lane form's: a sample small enough to start in the tail form is timed
+    # without it, and the batch's own setting is back afterwards.
+    print(f"[gpu] tuners without the tail form n={n}", flush=True)
+    from heyoka_amd import _lib
+
+    wl = W.cr3bp(n, log_t=(0.3, 0.8))
+    system = get_system(hy.taylor_decompose(wl.sys), 19)
+    made = []
+
+    class Recorded(_lib.Batch):
+        def __init__(self, *a):
+            super().__init__(*a)
+            made.append(self)
+
+    monkeypatch.setattr(AT._lib, "Batch", Recorded)
+    _, final = AT.measure(system, wl.state, wl.pars, wl.t_final, 2, 8)
+    assert len(made) == 1 and made[0].twin_launches() == 0
+    b = Recorded(system, n)
+    b.write_all(wl.state, wl.pars, np.zeros(n), np.zeros(n))
+    assert b.autotune(wl.t_final, tmp_path / "tune.txt")["rate"] > 0
+    assert b.twin_launches() == 0
+    b.propagate_until(wl.t_final)
+    assert b.twin_launches() == 1  # by default it starts there
+    np.testing.assert_array_equal(b.read(_lib.FIELD_STATE, wl.state.shape), final)
