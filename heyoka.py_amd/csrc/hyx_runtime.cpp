@@ -1149,6 +1149,9 @@ int hyx_batch_device_ptr(hyx_batch *b, int field, void **out)
     double *p;
     uint64_t count;
     if (int rc = field_info(b, field, &p, &count)) return rc;
+    // A small batch's last fill may still be on its way (hyx_batch_write_all).
+    if (b->hio_busy) HIPCHK(hipStreamSynchronize(b->stream));
+    b->hio_busy = false;
     *out = p;
     return 0;
 }

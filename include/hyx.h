@@ -143,7 +143,9 @@ int hyx_batch_write_all(hyx_batch *b, const double *state, const double *pars, c
                         const double *time_lo);
 int hyx_batch_read_all(hyx_batch *b, double *state, double *time_hi, double *time_lo, int64_t *outcome, double *min_h,
                        double *max_h, uint64_t *nsteps);
-/* Device pointer of a field (device-resident use, no copies). */
+/* Device pointer of a field (device-resident use, no copies). Waits for a fill under way. A caller that
+ * keeps the pointer and reads it on another stream after a later hyx_batch_write_all calls
+ * hyx_batch_sync (or this function) in between: that fill may return before its copy ends. */
 int hyx_batch_device_ptr(hyx_batch *b, int field, void **out);
 
 /* One adaptive step of every instance: step() / step(max_delta_t)

@@ -6,6 +6,7 @@ import pytest
 
 import heyoka_amd as hy
 from heyoka_amd import _lib, workloads
+from test_zz_no_alloc import D2H, _hip
 
 pytestmark = pytest.mark.gpu
 
@@ -70,3 +71,18 @@ def test_grid_faults_name_the_instance(row, col, msg):
     bad[row, col] = bad[row - 1, col] if row else 0.5
     with pytest.raises(_lib.HyxError, match=msg + f".*instance {col}|instance {col}.*" + msg):
         b.propagate_grid(bad)
+
+
+def test_device_pointer_of_a_filled_batch():
+    # From its second fill on a small batch returns before its copy ends; the device pointer waits
+    # for it, so that any stream reads the new values.
+    H = _hip()
+    n = 501
+    wl = workloads.cr3bp(n)
+    b = _lib.Batch(_lib.System(hy.taylor_decompose(wl.sys), 19), n)
+    for rep in range(4):
+        st = wl.state + rep
+        b.write_all(st, wl.pars, np.full(n, float(rep)), np.zeros(n))
+        out = np.empty_like(st)
+        assert H.hipMemcpy(out.ctypes.data, b.device_ptr(_lib.FIELD_STATE), out.nbytes, D2H) == 0
+        assert np.array_equal(out, st)
