@@ -2059,7 +2059,11 @@ std::string generate_group_prelude(const Sys &S, const GroupPlan &gp, int P, boo
     // scales get along with fit in 256 registers, and eight blocks in the 160 KB of LDS of a CU
     // (six bodies at order 19: 49 registers spill, outside the recurrences, and the step
     // takes 29 ms where it takes 36 ms at one wave per SIMD without spills; order 24 would
-    // spill histories).
+    // spill histories). Both sides of the line (order 20 for N bodies), 16,384 systems of 4 to 9 bodies
+    // to t = 40, time at two waves over time at one: order 12 0.99-1.02, 16 0.89-1.02, 19 0.73-0.94,
+    // 20 0.72-0.92, 21 0.71-0.95, 22 0.79-0.96, 24 0.87-1.67 (six bodies last; four do not fit the LDS
+    // condition from order 20 on). 301 systems, which leave SIMDs idle: 0.90-1.01 up to the line, up to
+    // 1.11 at order 22 and 1.48 at 24.
     const int hist = history_nodes(gp.tmpl) - (gen.raw_inputs ? nin : 0);
     if (derived && !E && 2 * hist * (P - 1) + 66 <= 256 &&
         (long)(flat + 16) * (64 / G) * 8 <= 20 * 1024)

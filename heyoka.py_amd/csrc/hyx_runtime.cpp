@@ -409,9 +409,9 @@ int build_sys(const uint32_t *ops, uint32_t n_words, const double *consts, uint3
             s.inst_per_block = 64u / (uint32_t)G;
         } else if (s.form == HYX_FORM_COMPACT && !(flags & HYX_FLAG_FORCE_COMPACT)) {
             // Systems too large for the register forms: the wave form when its LDS rows fit,
-            // 32 lanes per instance (measured on the J2 + variational ensemble: 5.9x the
-            // compact form's 2-lane tape in device memory; 16 lanes: 5.1x; 64 lanes: 3.2x),
-            // else 64.
+            // 32 lanes per instance (measured on 16,384 J2 + variational systems: 7.5e7 steps/s
+            // against 2.8e6 of the compact form's 2-lane tape in device memory; 16 lanes:
+            // 5.4e7; 64 lanes: 5.8e7), else 64.
             for (int G : {32, 64}) {
                 wave_src = hyx::generate_wave_prelude(s.S, (int)order, ha, G, s.has_events ? &s.E : nullptr,
                                                       (uint32_t)s.ev.dir.size(), split, why);
@@ -1348,7 +1348,11 @@ int run_propagation(hyx_batch *b, uint64_t max_steps, int mode, hyx_prop_res *re
             // 200 time units of the CR3BP: 1.26 ms per 16,384 instances in the quad form, 3.18 ms
             // per 65,536 in the lane form, so 2.5 against 3.2 ms at the line, 3.8 for the quad's next
             // round). Kernel time, started in the lane form and now: 200 orbits over 50 time
-            // units 0.62 -> 0.38 ms, 5,000 over 20 0.35 -> 0.19 ms, 32,768 over 20 0.43 -> 0.37 ms.
+            // units 0.62 -> 0.38 ms, 5,000 over 20 0.35 -> 0.19 ms, 32,768 over 20 0.43 -> 0.37 ms. In
+            // the twin form (two lanes per instance, one round up to the line) of three systems, the
+            // CR3BP, the same with a perturbed x and two coupled sines, over 50 time units: 4,096
+            // 0.60 -> 0.43, 0.63 -> 0.46 and 0.85 -> 0.64 ms, 32,768 0.84 -> 0.52, 1.07 -> 0.55 and
+            // 1.41 -> 0.77 ms.
             const uint64_t direct = b->tail_auto ? std::max<uint64_t>(b->tail_min, (uint64_t)b->n_cu * 4 * 64 / 2) : b->tail_min;
             if (N <= direct) {
                 HIPCHK(hipEventRecord(b->evt, b->stream));

@@ -396,7 +396,9 @@ class taylor_adaptive_batch:
         elif write_tc:
             self._read_tc()
         # One enum member per outcome, not one lookup per lane (a step of 20,000 lanes with its
-        # coefficients, these read in place too: 7.7 -> 2.7 ms).
+        # coefficients, these read in place too: 14.5 -> 8.9 ms call after call, where the
+        # interpreter's garbage collections over the tuples are 6 ms of either; one call alone
+        # 7.7 -> 2.7 ms).
         ocs = oc.tolist()
         names = {v: _outcome(v) for v in set(ocs)}
         self._hyx_step_res = list(zip(map(names.__getitem__, ocs), h.tolist()))
