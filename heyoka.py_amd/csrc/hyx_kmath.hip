@@ -9,7 +9,7 @@
 // of them (logarithm and exponential in extended precision, every special case). Measured when
 // they came in, with pow() and with these functions: four pendulums to t = 100 1.09 -> 0.80 ms,
 // 65,536 six-body systems to t = 10 56.2 -> 52.6 ms. VALU instructions of hyx_step_k, with pow() and
-// now: pendulum 1,086 and 785, planar CR3BP in the quad form 1,797 and 1,556.
+// now: pendulum 1,086 and 784, planar CR3BP in the quad form 1,797 and 1,555.
 
 template <int R>
 __device__ __forceinline__ double hyx_ipow(double y)
@@ -35,10 +35,7 @@ template <int R>
 __device__ __forceinline__ double hyx_root(double rnum, double den)
 {
 #pragma STDC FP_CONTRACT OFF
-    // (By a select here: a return at the end becomes a branch around the iterations, and the four
-    // pendulums' kernel takes 0.63 instead of 0.60 ms.)
-    const double q0 = den * rnum;
-    const double q = q0 <= 0x1p-1024 ? 0.0 : q0;
+    const double q = den * rnum;
 #ifdef __AMDGCN__
     const double m = __builtin_amdgcn_frexp_mant(q);
     const float l = __builtin_amdgcn_logf((float)m), ef = (float)__builtin_amdgcn_frexp_exp(q);
@@ -59,8 +56,12 @@ __device__ __forceinline__ double hyx_root(double rnum, double den)
     double y = (double)y0;
     y = __builtin_fma(y * (1.0 / R), __builtin_fma(-qs, hyx_ipow<R>(y), 1.0), y);
     y = __builtin_fma(y * (1.0 / R), __builtin_fma(-qs, hyx_ipow<R>(y), 1.0), y);
-    // At either end the start is the value.
-    return (q == 0.0 || q == __builtin_inf()) ? (double)y0 : ldexp(y, -ei);
+    // Beyond the largest double: a scale that overflows. (One select of an integer: flushing q to
+    // zero first takes a step of 200 CR3BP orbits 2.5 % longer, and a return at the end, which becomes
+    // a branch around the iterations, one of four pendulums 5 %.)
+    const double r = ldexp(y, q <= 0x1p-1024 ? 4096 : -ei);
+    // q = 0 or inf: the start is the value.
+    return (q == 0.0 || q == __builtin_inf()) ? (double)y0 : r;
 }
 
 // s ~ x^(-1/2) to about one ulp, and its correction: p + pl = s^2 exactly, and
